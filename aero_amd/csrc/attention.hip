@@ -3,12 +3,14 @@
 // softmax (src/tensor.cpp:167-178) and the KV cache vector quantisers
 // (include/aero/kv.hpp:62-103, src/kv.cpp:13-46).
 //
-// Two attention kernels share one plan. Keys are split into chunks when the
+// The attention kernels share one plan. Keys are split into chunks when the
 // query tiles alone do not fill the chip (decode: one query, many keys); each
 // chunk's (max m, sum l, accumulator) is merged by attn_combine_kernel.
 //  * attn_mfma_kernel (head_dim == value_dim in {64, 128, 256}): scores and
 //    the value sum on the fp32 matrix cores, a wave per 16-key tile, the
 //    workgroup's four waves sharing one 16-query tile.
+//  * attn_split_kernel (attn_split.hpp): the same head dims, prompts over an
+//    fp32 cache that fill the chip, on the fp16 matrix cores by split operands.
 //  * attn_kernel (any other width up to 256): 16-lane groups own a key, the
 //    dot product is reduced with lane shuffles, four query vectors a
 //    workgroup.
@@ -26,6 +28,7 @@
 #include "aero_hip.h"
 
 #include <cmath>
+#include <type_traits>
 
 namespace aero {
 
@@ -1009,6 +1012,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
     merge_tile<Tile, D, MERGE_OUT>(p, m, ls, acc, tile, n_vec, chunk, kh, wave, g, c);
 }
 
+#include "attn_split.hpp"
+
 // Merge the chunks' (m, l, acc) of one (token, head) row per workgroup. Thread
 // (part q, element d) loads (m, l, acc[d]) of chunks q, q + P, ... all at once
 // (clamped indices, no branch between the loads), merges them in registers,
@@ -1214,7 +1219,19 @@ AttnKernel pick_f16(int dt, int D, bool merge_out, bool kpos) {
                    : (dt == 2 ? pick_f16_dt<2>(D, merge_out, kpos) : nullptr);
 }
 
+AttnKernel pick_split(int D, bool kpos) {
+    switch (D) {
+    case 64: return kpos ? attn_split_kernel<64, true> : attn_split_kernel<64, false>;
+    case 128: return kpos ? attn_split_kernel<128, true> : attn_split_kernel<128, false>;
+    case 256: return kpos ? attn_split_kernel<256, true> : attn_split_kernel<256, false>;
+    default: return nullptr;
+    }
+}
+
+int split_waves(int D) { return D == 256 ? SplitCfg<256>::NW : SplitCfg<128>::NW; }
+
 struct AttnPlan {
+    bool split;            // fp32 cache on the fp16 matrix cores (attn_split_kernel)
     bool mfma;
     bool f16;              // integer caches on the fp16 matrix cores (attn_f16_kernel)
     int E;                 // VALU kernel: elements per lane
@@ -1262,7 +1279,40 @@ bool attn_plan(int64_t n_q, int64_t n_head, int64_t n_head_kv, int64_t head_dim,
     // the fp16 kernel addresses a chunk of one kv head with 32-bit offsets
     const int64_t vec_bytes = head_dim * (kv_dt == 1 ? 8 : 4) / 8;
     if (pl.f16 && cl * n_head_kv * vec_bytes >= (int64_t(1) << 31)) pl.f16 = false;
+    pl.split = false;
     return true;
+}
+
+// Whether a call that attn_mfma_kernel would take as one chunk goes to
+// attn_split_kernel: fp32 caches, and enough workgroups (128 query vectors of
+// a kv head each, one a CU) that the chip is half full, or more than a
+// quarter full over long key ranges, where the split of the keys is paid back.
+// Measured on MI355X, fp32-step kernel / this one in us, causal prompts
+// unless noted: 8 kv heads of dim 128, 32 heads: 104 workgroups (400 tokens)
+// 35.0 / 36.8, after 1000 cached keys 141 / 90; 176 (700 tokens) 76.0 / 52.7;
+// 512 (2048 tokens) 463 / 150; dim 64: 104 workgroups 19.4 / 25.1, after 1000
+// keys 84.6 / 51.7; 176: 44.8 / 33.4. Two kv heads of dim 64, 14 heads, 78
+// workgroups: 25.7 / 31.2, after 1000 keys 69.8 / 60.1. Dim 256, 88
+// workgroups: 152 / 179 (1400 tokens, 700 keys a query), after 1000 keys
+// 309 / 294 and in a window of 1024 208 / 150. Below 72 workgroups the
+// fp32-step kernel, which also splits the keys, is the faster one for most
+// sizes (64 workgroups of dim 128, 256 tokens: 18.2 / 26.8).
+void plan_split(int64_t n_q, int64_t n_head, int64_t n_head_kv, int64_t head_dim, int64_t n_kv,
+                int window, int kv_dt, AttnPlan& pl) {
+    const int use = tune("attn_split", 1);   // 2: whatever the sizes
+    const int64_t grid_z = (n_q * (n_head / n_head_kv) + kSplitVecs - 1) / kSplitVecs;
+    const int64_t wgs = n_head_kv * grid_z;
+    int64_t mean = std::max<int64_t>(n_kv - n_q / 2, 1);   // keys a query, causal
+    if (window > 0) mean = std::min<int64_t>(mean, window);
+    if (!pl.mfma || kv_dt != 0 || use == 0 ||
+        (use == 1 && (pl.n_chunks != 1 || !(wgs >= 128 || (wgs >= 72 && mean >= 1000)))) ||
+        // (32-bit key indices and offsets within a key tile)
+        n_kv >= (int64_t(1) << 30) || n_head_kv * head_dim * 4 * 128 >= (int64_t(1) << 31))
+        return;
+    pl.split = true;
+    pl.grid_z = grid_z;
+    pl.chunk_len = n_kv;
+    pl.n_chunks = 1;
 }
 
 // ------------------------------------------------------------ KV writes
@@ -1398,16 +1448,18 @@ bool attention_dev(const float* q, int kv_dt, const void* k, const float* k_scal
         set_error("attention: grid too large");
         return false;
     }
+    plan_split(n_q, n_head, n_head_kv, head_dim, n_kv, window, kv_dt, pl);
     AttnParams p{q, k, k_scale, v, v_scale, out, static_cast<float*>(workspace), qpos, kpos,
                  n_q, n_head, n_head_kv, head_dim, value_dim, n_kv,
                  (int)(n_head / n_head_kv), window, scale, pl.chunk_len, pl.n_chunks};
     const bool one = pl.n_chunks == 1;
-    AttnKernel kern = pl.f16 ? pick_f16(kv_dt, (int)head_dim, one, kpos != nullptr)
+    AttnKernel kern = pl.split ? pick_split((int)head_dim, kpos != nullptr)
+                      : pl.f16 ? pick_f16(kv_dt, (int)head_dim, one, kpos != nullptr)
                       : pl.mfma ? pick_mfma(kv_dt, (int)head_dim, one)
                                 : pick_attn(kv_dt, pl.E, one);
-    if (!launch(pl.f16 ? "attn_f16_kernel" : (pl.mfma ? "attn_mfma_kernel" : "attn_kernel"), kern,
+    if (!launch(pl.split ? "attn_split_kernel" : pl.f16 ? "attn_f16_kernel" : (pl.mfma ? "attn_mfma_kernel" : "attn_kernel"), kern,
                 dim3((unsigned)pl.n_chunks, (unsigned)n_head_kv, (unsigned)pl.grid_z),
-                dim3(64 * kAttnWaves), 0, s, p))
+                dim3(pl.split ? 64 * split_waves((int)head_dim) : 64 * kAttnWaves), 0, s, p))
         return false;
     // (value widths of a multiple of 4 up to 256 here: DV / 4 <= 512 lanes)
     const bool c4 = value_dim % 4 == 0 && aligned16(workspace) && aligned16(out) &&

@@ -1,0 +1,722 @@
+// Prefill attention over an fp32 KV cache on the fp16 matrix cores (included
+// by attention.hip after its fp16 helpers).
+//
+// v_mfma_f32_32x32x16_f16: lane l (n = l % 32, h = l / 32) supplies
+// A[n][8h..8h+7] and B[8h..8h+7][n] and receives D[8j + 4h + r][n], j, r =
+// 0..3, in element 4j + r. Everything is computed transposed, so a lane's
+// column is one query throughout and the softmax state, its rescaling and the
+// output rows are lane-local:
+//  * S^T = K Q^T: A = 32 keys x 16 dimensions, B = the wave's 32 queries;
+//  * O^T += V^T P^T: A = 32 value dimensions x 16 keys, B = the
+//    probabilities as the scores' accumulator holds them (k-slots 8h + 4b + r
+//    of step s are key 16s + 8b + 4h + r, and V^T is stored in that order).
+// Four waves share the keys of a tile and own 32 query vectors each.
+//
+// Arithmetic: q (a power of two per query), K and V (a power of two per
+// wave's share of a tile, KW keys) are scaled to below 2^14 and split into
+// two fp16 parts, hi = fp16(v), lo = fp16(v - hi): 22 bits, and 2^-39 of the
+// block's largest below that. Products are hi hi + hi lo + lo hi, exact,
+// added in fp32 by the matrix cores. The probabilities (<= 1, against a
+// reference max m that is a whole number of log2 units) are split the same
+// way, in units of 2^(ev - E + 14), ev the exponent of the key's V block and E
+// that of the sums; the sums take each step's product with one fma, which
+// carries the change of m and E. Keys that no query of the workgroup
+// keeps become zeros, so what lies in them does not touch the scales.
+// What the split cannot carry is done again in plain fp32 by the wave that
+// owns the rows (attn_rows_plain, about 30 times slower): an infinity (a split
+// makes a NaN of it), sums that are not finite (a NaN among the values reaches
+// queries that do not keep its key), value blocks whose exponents differ by
+// more than 15 or keys and queries whose products pass 2^14 (a small one next
+// to them would keep less than fp32's 24 bits).
+//
+// Shape. A workgroup owns 128 query vectors of one kv head (32 a wave). At
+// head dims 64 and 128 eight waves walk 128 / 64 keys a step, two waves a
+// query group, each on half of the sub-tiles (their sums meet in LDS at the
+// end): a workgroup's walk, which bounds the call where the causal triangle
+// leaves some twice the mean, is half as long as with four. At 256 the
+// query's parts and the sums take 256 registers, so four waves with the
+// register file to themselves walk 32 keys. K and V are split once a
+// workgroup into LDS (double-buffered; the split runs between the scores'
+// matrix steps, the next loads between the value sum's).
+// What bounds it: per 64 keys and CU at head dim 128 3072 cycles of matrix
+// steps a SIMD, about 2600 of LDS, about 2400 of vector instructions a SIMD
+// and a step takes about 7500: two waves a SIMD (all 256 registers each) do
+// not overlap them fully. Against attn_mfma_kernel, whose fp32 steps run at a
+// sixteenth of the fp16 rate, on MI355X, 2048 causal tokens: 32 / 8 heads of
+// dim 128 463 -> 150 us (229 TFLOP/s by the useful products), of dim 64
+// 256 -> 85 us, 8 / 4 heads of dim 256 in a window of 1024 222 -> 146 us.
+// Error against float64 (2-norm) at those sizes: 4.0e-7 -> 2.9e-7, 3.3e-7 ->
+// 2.5e-7, 5.0e-7 -> 3.5e-7.
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+
+template <int D>
+struct SplitCfg {
+    static constexpr int NW = D == 256 ? 4 : 8;       // waves
+    static constexpr int GK = NW / 4;                 // waves on the same queries
+    static constexpr int KT = D == 64 ? 128 : (D == 128 ? 64 : 32);   // keys a tile
+    static constexpr int SUBS = KT / 32;
+    static constexpr int KW = KT / NW;                // keys a wave converts
+    static constexpr int LK = D / 8;                  // K: lanes a key (8 dimensions each)
+    static constexpr int PK = 64 / LK, NK = KW / PK;  // keys a pass, passes
+    static constexpr int CV = D == 256 ? 2 : 1;       // V: column passes (2 dimensions a lane)
+    static constexpr int NP = NK + 2 * CV;            // pieces of 8 elements a lane converts
+    static constexpr int OW = KW / 8;                 // key octets a wave converts
+    static constexpr int KP = D + 8;                  // K row pitch, halves
+    static constexpr int VP = 40;                     // V^T row pitch, halves (32 keys + 16 B)
+    static constexpr int KPART = KT * KP, VPART = SUBS * D * VP;
+    static constexpr int BUF = 2 * (KPART + VPART);   // halves
+};
+
+// two fp32 values (already scaled) as fp16 hi and lo pairs: lo from one
+// mixed-precision fma an element (v_fma_mix_f32 issues in half the time of
+// v_fma_mixlo_f16, which the compiler prefers) and a packed conversion
+__device__ __forceinline__ void split_pair(float a, float b, h2& hi, h2& lo) {
+    hi = __builtin_convertvector((v2f){a, b}, h2);
+    float x, y;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(x) : "v"(hi), "v"(a));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+        : "=v"(y) : "v"(hi), "v"(b));
+    lo = __builtin_convertvector((v2f){x, y}, h2);
+}
+
+// max of three (magnitudes): v_max3_f32 directly, without the compiler's
+// quieting of each operand (a NaN is ignored; it shows in the results)
+__device__ __forceinline__ float max3(float a, float b, float c) {
+    asm("v_max3_f32 %0, %0, %1, %2" : "+v"(a) : "v"(b), "v"(c));
+    return a;
+}
+__device__ __forceinline__ float max3_abs(float a, float b, float c) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(a) : "v"(b), "v"(c));
+    return a;
+}
+
+// the largest a and b over each 16-lane row, in every lane of it (a DPP
+// operand may be read two instructions after it is written)
+__device__ __forceinline__ void row_max2(float& a, float& b) {
+    asm("s_nop 1\n"
+        "v_max_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0xf\n"
+        "s_nop 0\n"
+        "v_max_f32_dpp %0, %0, %0 row_ror:4 row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %1, %1, %1 row_ror:4 row_mask:0xf bank_mask:0xf\n"
+        "s_nop 0\n"
+        "v_max_f32_dpp %0, %0, %0 row_ror:2 row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %1, %1, %1 row_ror:2 row_mask:0xf bank_mask:0xf\n"
+        "s_nop 0\n"
+        "v_max_f32_dpp %0, %0, %0 row_ror:1 row_mask:0xf bank_mask:0xf\n"
+        "v_max_f32_dpp %1, %1, %1 row_ror:1 row_mask:0xf bank_mask:0xf\n"
+        "s_nop 1"
+        : "+v"(a), "+v"(b));
+}
+// the largest a and b over the wave, wave-uniform
+__device__ __forceinline__ void wave_max2(float& a, float& b) {
+    row_max2(a, b);
+    asm("v_max_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n"
+        "v_max_f32_dpp %1, %1, %1 row_bcast:15 row_mask:0xa bank_mask:0xf\n"
+        "s_nop 0\n"
+        "v_max_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n"
+        "v_max_f32_dpp %1, %1, %1 row_bcast:31 row_mask:0xc bank_mask:0xf\n"
+        "s_nop 1"
+        : "+v"(a), "+v"(b));
+    a = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), 63));
+    b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, b), 63));
+}
+
+// e with |x| < 2^e for a block's largest |x|, clamped so that 2^(14 - e) and
+// 2^(e - 14) are normal (129 for an infinity)
+__device__ __forceinline__ int block_exp(float amax) {
+    return max((int)(__builtin_bit_cast(uint32_t, amax) >> 23) - 126, -112);
+}
+
+// One wave's n query vectors u0.. of kv head kh over keys [j0, j1), one after
+// the other in plain fp32: the fallback for operands that hold infinities.
+// 64 keys a step, a lane a key for the scores, a lane D / 64 dimensions for
+// the value sum.
+template <int D>
+__device__ __forceinline__ void attn_rows_plain(const AttnParams& p, int64_t u0, int n, int kh,
+                                                int j0, int j1) {
+    constexpr int E = D / 64;
+    const int lane = threadIdx.x & 63;
+    const float* kg = static_cast<const float*>(p.k);
+    const float* vg = static_cast<const float*>(p.v);
+    for (int i = 0; i < n; ++i) {
+        const int64_t u = u0 + i, t = u / p.rep;
+        const int64_t row = t * p.n_head + (int64_t)kh * p.rep + u % p.rep;
+        const int64_t qp = p.qpos ? (int64_t)p.qpos[t] : t;
+        const float* q = p.q + row * D;
+        float m = -INFINITY, l = 0.0f, acc[E];
+        for (int e = 0; e < E; ++e) acc[e] = 0.0f;
+        for (int jb = j0; jb < j1; jb += 64) {
+            const int j = min(jb + lane, j1 - 1);
+            const float* kv = kg + ((int64_t)j * p.n_head_kv + kh) * D;
+            float s = 0.0f;
+#pragma unroll 4
+            for (int d = 0; d < D; ++d) s = __builtin_fmaf(q[d], kv[d], s);
+            const int64_t kp = p.kpos ? (int64_t)p.kpos[j] : j;
+            const bool keep = jb + lane < j1 && key_kept(kp, qp, p.window);
+            s = keep ? s * p.scale : -INFINITY;
+            float mn = fmaxf(m, s);
+            for (int off = 32; off >= 1; off >>= 1) mn = fmaxf(mn, __shfl_xor(mn, off));
+            const float alpha = (m == -INFINITY) ? 0.0f : expf(m - mn);
+            const float pr = (s == -INFINITY) ? 0.0f : expf(s - mn);
+            l = l * alpha + group_sum<64>(pr);
+            for (int e = 0; e < E; ++e) acc[e] *= alpha;
+            for (uint64_t left = __ballot(keep); left != 0; left &= left - 1) {
+                const int x = __ffsll((unsigned long long)left) - 1;
+                const float w = __shfl(pr, x);
+                const float* vv = vg + ((int64_t)(jb + x) * p.n_head_kv + kh) * D;
+                for (int e = 0; e < E; ++e)
+                    acc[e] = __builtin_fmaf(w, vv[64 * e + lane], acc[e]);
+            }
+            m = mn;
+        }
+        for (int e = 0; e < E; ++e) p.out[row * D + 64 * e + lane] = acc[e] / fmaxf(l, 1e-30f);
+    }
+}
+
+constexpr float kLog2eLo = 1.92596299e-8f;   // log2(e) - kLog2e
+constexpr int kNoMax = -(1 << 28);     // no key kept yet
+constexpr int kSplitVecs = 128;   // query vectors a workgroup
+
+template <int D, bool KPOS>
+__global__ __launch_bounds__(64 * SplitCfg<D>::NW)
+__attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(AttnParams p) {
+    using C = SplitCfg<D>;
+    constexpr int NT = D / 32, NS = D / 16;
+    __shared__ __attribute__((aligned(16))) _Float16 smem[2][C::BUF];
+    __shared__ float s_kf[2][C::NW];   // 2^(e - 14) of each wave's keys
+    __shared__ int s_ev[2][C::NW];     // exponent of each wave's values
+    __shared__ int s_bad;              // operands that the split would not carry
+    __shared__ int s_eq;               // the largest query exponent
+    __shared__ int s_er[2][C::NW];     // each wave's value exponents: smallest, largest
+    __shared__ int32_t s_kp[2][C::KT];
+    __shared__ int32_t s_q[2][4];
+    __shared__ float s_qe[kSplitVecs];   // 2^(e - 14) of each query
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int qg = wave & 3, gk = wave >> 2;
+    const int n = lane & 31, h = lane >> 5;
+    const int kh = blockIdx.y;
+    const uint32_t n_vec = (uint32_t)p.n_q * (uint32_t)p.rep;
+    const uint32_t tile = gridDim.z - 1 - blockIdx.z;
+    const int n_kv = (int)p.n_kv;
+
+    // the lane's query vector: token tq, head kh * rep + u % rep
+    const uint32_t u = tile * kSplitVecs + qg * 32 + n;
+    const bool qok = u < n_vec;
+    const uint32_t uc = qok ? u : n_vec - 1;
+    const uint32_t tq = uc / (uint32_t)p.rep;
+    const uint32_t qrow = tq * (uint32_t)p.n_head + (uint32_t)(kh * p.rep) + uc % (uint32_t)p.rep;
+    const int32_t qp = p.qpos ? p.qpos[tq] : (int32_t)tq;
+
+    // The wave's share of its group's queries (32 / GK rows, whole rows at a
+    // time), loaded before the positions are known.
+    constexpr int LQ = D / 4, PQ = 64 / LQ, NQ = 32 / C::GK / PQ;
+    const int r0 = gk * (32 / C::GK) + lane / LQ, lq = lane % LQ;
+    v4f f[NQ];
+#pragma unroll
+    for (int x = 0; x < NQ; ++x) {
+        const uint32_t row = (uint32_t)__shfl((int)qrow, r0 + PQ * x);
+        f[x] = *reinterpret_cast<const v4f*>(p.q + (int64_t)row * D + 4 * lq);
+    }
+
+    int32_t qmin = qp, qmax = qp;
+#pragma unroll
+    for (int off = 16; off >= 1; off >>= 1) {
+        qmin = min(qmin, __shfl_xor(qmin, off));
+        qmax = max(qmax, __shfl_xor(qmax, off));
+    }
+    qmin = __builtin_amdgcn_readfirstlane(qmin);
+    qmax = __builtin_amdgcn_readfirstlane(qmax);
+    if (lane == 0 && gk == 0) {
+        s_q[0][qg] = qmin;
+        s_q[1][qg] = qmax;
+        if (qg == 0) {
+            s_bad = 0;
+            s_eq = -1000;
+        }
+    }
+    __syncthreads();
+    const int32_t wmin = __builtin_amdgcn_readfirstlane(
+        min(min(s_q[0][0], s_q[0][1]), min(s_q[0][2], s_q[0][3])));
+    const int32_t wmax = __builtin_amdgcn_readfirstlane(
+        max(max(s_q[1][0], s_q[1][1]), max(s_q[1][2], s_q[1][3])));
+
+    // key tiles [i_lo, i_hi) that can hold kept keys (as attn_mfma_kernel)
+    int i_lo = 0, i_hi = (n_kv + C::KT - 1) / C::KT;
+    if constexpr (!KPOS) {
+        i_hi = (int)min<int64_t>(i_hi, max<int64_t>(0, ((int64_t)wmax + C::KT) / C::KT));
+        if (p.window > 0)
+            i_lo = (int)max<int64_t>(0, ((int64_t)wmin - p.window + 1) / C::KT);
+    }
+
+    // A tile on its way to LDS, through buffer descriptors of the tile (keys
+    // at or past n_kv read as zeros): of a wave's KW keys, lane (lane / LK,
+    // lane % LK) takes dimensions 4lk .. +3 and D/2 + 4lk .. +3 of key PK * pass
+    // + lane / LK of K (adjacent in LDS, as in q's rows there: a dot product
+    // does not depend on the order of its terms), and 2 dimensions of the 8 keys of one octet of V (octet o of a sub-tile: keys
+    // 16(o / 2) + 4(o % 2) + r and 8 more, the order of its 16 bytes of V^T).
+    const int lk = lane % C::LK, pk = lane / C::LK;
+    const int vo = D == 64 ? wave * 2 + (lane >> 5) : wave;
+    const int vd = D == 64 ? 2 * (lane & 31) : 2 * lane;
+    const int vk = 32 * (vo >> 2) + 16 * ((vo >> 1) & 1) + 4 * (vo & 1);
+    const uint32_t kstride = (uint32_t)(p.n_head_kv * D * 4);
+    const uint32_t koff = (uint32_t)(wave * C::KW + pk) * kstride + (uint32_t)lk * 16u;
+    const uint32_t voff = (uint32_t)vk * kstride + (uint32_t)vd * 4u;
+    const uint8_t* kbase = reinterpret_cast<const uint8_t*>(static_cast<const float*>(p.k) +
+                                                            (int64_t)kh * D);
+    const uint8_t* vbase = reinterpret_cast<const uint8_t*>(static_cast<const float*>(p.v) +
+                                                            (int64_t)kh * D);
+    v4f kr[C::NK][2];
+    v2f vr[C::CV][8];
+    int32_t kpr = 0;
+    // a descriptor of the keys from key0 on (its size: the tile at most)
+    auto rsrc = [&](const uint8_t* base, int key0) __attribute__((always_inline)) {
+        const int left = min(n_kv - key0, C::KT);
+        return __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint8_t*>(base) + (int64_t)key0 * kstride, 0,
+            left > 0 ? (int)((uint32_t)(left - 1) * kstride + D * 4) : 0, kBufferDword3);
+    };
+    // load x of a tile: 2 NK of K, 8 CV of V (a descriptor each: the lane's
+    // offsets are the same for all, so no registers hold the others)
+    constexpr int NL = 2 * C::NK + 8 * C::CV;
+    auto load1 = [&](int i, int x) __attribute__((always_inline)) {
+        if (x < 2 * C::NK) {
+            kr[x >> 1][x & 1] = __builtin_bit_cast(
+                v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                         rsrc(kbase, i * C::KT + (x >> 1) * C::PK), (int)(koff + 2u * D * (x & 1)),
+                         0, 0));
+        } else {
+            const int e = (x - 2 * C::NK) & 7, c = (x - 2 * C::NK) >> 3;
+            vr[c][e] = __builtin_bit_cast(
+                v2f, __builtin_amdgcn_raw_buffer_load_b64(
+                         rsrc(vbase, i * C::KT + (e >> 2) * 8 + (e & 3)), (int)(voff + 512u * c),
+                         0, 0));
+        }
+        if constexpr (KPOS) {   // (lane's key of the wave's KW)
+            if (x == 0)
+                kpr = p.kpos[min(i * C::KT + wave * C::KW + (lane & (C::KW - 1)), n_kv - 1)];
+        }
+    };
+    auto load = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int x = 0; x < NL; ++x) load1(i, x);
+    };
+    // the loaded tile (i), on its way to buffer b: keys that nothing keeps
+    // zeroed, the scales
+    float fk, fv;
+    int ek_lim = 0, ev_lo = 1000, ev_hi = -1000;
+    auto scales = [&](int b, int i) __attribute__((always_inline)) {
+        const int first = i * C::KT + wave * C::KW;
+        // keys of the tile that no query of the workgroup keeps become zeros
+        auto visible = [&](int key, int32_t kp) __attribute__((always_inline)) {
+            return key < n_kv && kp <= wmax && (p.window <= 0 || (int64_t)wmin - kp < p.window);
+        };
+        if constexpr (KPOS) {
+            if (lane < C::KW) s_kp[b][wave * C::KW + lane] = kpr;
+        }
+        if (KPOS || (i + 1) * C::KT - 1 > wmax ||
+            (p.window > 0 && (int64_t)wmin - i * C::KT >= p.window)) {
+            asm volatile("");
+#pragma unroll
+            for (int x = 0; x < C::NK; ++x) {
+                const int key = first + x * C::PK + pk;
+                int32_t kp = key;
+                if constexpr (KPOS) kp = __shfl(kpr, x * C::PK + pk);
+                const bool vis = visible(key, kp);
+#pragma unroll
+                for (int y = 0; y < 8; ++y)
+                    kr[x][y >> 2][y & 3] = vis ? kr[x][y >> 2][y & 3] : 0.0f;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int key = i * C::KT + vk + (e >> 2) * 8 + (e & 3);
+                int32_t kp = key;
+                if constexpr (KPOS) kp = p.kpos[min(key, n_kv - 1)];
+                const bool vis = visible(key, kp);
+#pragma unroll
+                for (int x = 0; x < C::CV; ++x) {
+                    vr[x][e].x = vis ? vr[x][e].x : 0.0f;
+                    vr[x][e].y = vis ? vr[x][e].y : 0.0f;
+                }
+            }
+        }
+        float ak = 0.0f, av = 0.0f;
+#pragma unroll
+        for (int x = 0; x < C::NK; ++x)
+#pragma unroll
+            for (int y = 0; y < 8; y += 2)
+                ak = max3_abs(ak, kr[x][y >> 2][y & 3], kr[x][y >> 2][(y & 3) + 1]);
+#pragma unroll
+        for (int x = 0; x < C::CV; ++x)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) av = max3_abs(av, vr[x][e].x, vr[x][e].y);
+        wave_max2(ak, av);
+        const int ek = block_exp(ak), ev = block_exp(av);
+        if (lane == 0) {
+            s_kf[b][wave] = pow2i(ek - 14);
+            s_ev[b][wave] = ev;
+            if (ev > 128 || ek > ek_lim) s_bad = 1;
+        }
+        if (ev > -112) {
+            ev_lo = min(ev_lo, ev);
+            ev_hi = max(ev_hi, ev);
+        }
+        fk = pow2i(14 - ek);
+        fv = pow2i(14 - ev);
+    };
+    // pair y (of 4) of piece x (8 elements) of the loaded tile's split; the
+    // piece goes to buffer b with its last pair
+    h2 chi[4], clo[4];
+    auto convert = [&](int b, int x, int y) __attribute__((always_inline)) {
+        _Float16* o;
+        int part;
+        if (x < C::NK) {
+            split_pair(kr[x][y >> 1][2 * (y & 1)] * fk, kr[x][y >> 1][2 * (y & 1) + 1] * fk,
+                       chi[y], clo[y]);
+            o = smem[b] + (wave * C::KW + pk + x * C::PK) * C::KP + 8 * lk;
+            part = C::KPART;
+        } else {
+            // V^T row (a dimension): the octet's 16 bytes, swizzled by the
+            // dimension so that a column of rows covers the banks
+            const int c = (x - C::NK) >> 1, d = (x - C::NK) & 1;
+            split_pair(vr[c][2 * y][d] * fv, vr[c][2 * y + 1][d] * fv, chi[y], clo[y]);
+            o = smem[b] + 2 * C::KPART + ((vo >> 2) * D + vd + 128 * c + d) * C::VP +
+                ((vo & 3) ^ ((vd >> 4) & 3)) * 8;
+            part = C::VPART;
+        }
+        if (y == 3) {
+            *reinterpret_cast<uint4*>(o) =
+                make_uint4(h2_u32(chi[0]), h2_u32(chi[1]), h2_u32(chi[2]), h2_u32(chi[3]));
+            *reinterpret_cast<uint4*>(o + part) =
+                make_uint4(h2_u32(clo[0]), h2_u32(clo[1]), h2_u32(clo[2]), h2_u32(clo[3]));
+        }
+    };
+
+    if (i_lo < i_hi) load(i_lo);
+
+    // the positions the lane's query keeps: klo .. qp (khi without key
+    // positions, where the key's place bounds them too)
+    const int32_t klo = p.window > 0 ? (int32_t)max<int64_t>((int64_t)qp - p.window + 1,
+                                                             KPOS ? INT32_MIN : 0)
+                                     : (KPOS ? INT32_MIN : 0);
+    const int32_t klo_max =
+        p.window > 0 ? (int32_t)max<int64_t>((int64_t)qmax - p.window + 1, 0) : 0;
+    const int32_t khi = max(min(qp, n_kv - 1), -1);
+
+    // the query's parts, times scale * log2(e) (its product with two floats,
+    // so that the scores' factor c is a power of two), through LDS into the
+    // matrix operand's order: dimensions 16st + 8h .. +7 of step st.
+    h8 qhi[NS], qlo[NS];
+    float qsc;
+    {
+        constexpr int QPART = kSplitVecs * C::KP;
+        static_assert(4 * QPART <= (int)sizeof(smem), "query staging");
+        _Float16* qs = &smem[0][0];
+        const float c0 = p.scale * kLog2e;
+        const float c1 = __builtin_fmaf(p.scale, kLog2e, -c0) + p.scale * kLog2eLo;
+        float amax[NQ];
+#pragma unroll
+        for (int x = 0; x < NQ; ++x) amax[x] = max3_abs(max3_abs(0.0f, f[x][0], f[x][1]), f[x][2], f[x][3]);
+#pragma unroll
+        for (int x = 0; x < NQ; x += 2) {
+            row_max2(amax[x], amax[x + 1]);
+#pragma unroll
+            for (int y = x; y < x + 2; ++y) {
+                if constexpr (LQ >= 32) amax[y] = fmaxf(amax[y], __shfl_xor(amax[y], 16));
+                if constexpr (LQ >= 64) amax[y] = fmaxf(amax[y], __shfl_xor(amax[y], 32));
+            }
+        }
+#pragma unroll
+        for (int x = 0; x < NQ; ++x) {
+            const int eq = block_exp(amax[x] * fabsf(c0) * 1.0001f);
+            const float f0 = pow2i(14 - eq);
+            if (lq == 0) {
+                s_qe[qg * 32 + r0 + PQ * x] = pow2i(eq - 14);
+                if (eq > 128) s_bad = 1;
+                atomicMax(&s_eq, eq);
+            }
+            h2 hi[2], lo[2];
+#pragma unroll
+            for (int y = 0; y < 4; ++y)
+                f[x][y] = __builtin_fmaf(f[x][y], c0, f[x][y] * c1) * f0;
+            split_pair(f[x][0], f[x][1], hi[0], lo[0]);
+            split_pair(f[x][2], f[x][3], hi[1], lo[1]);
+            _Float16* o = qs + (qg * 32 + r0 + PQ * x) * C::KP + 8 * (lq % (LQ / 2)) +
+                          4 * (lq / (LQ / 2));
+            *reinterpret_cast<uint2*>(o) = make_uint2(h2_u32(hi[0]), h2_u32(hi[1]));
+            *reinterpret_cast<uint2*>(o + QPART) = make_uint2(h2_u32(lo[0]), h2_u32(lo[1]));
+        }
+        __syncthreads();
+        const _Float16* qf = qs + (qg * 32 + n) * C::KP + 8 * h;
+#pragma unroll
+        for (int st = 0; st < NS; ++st) {
+            qhi[st] = *reinterpret_cast<const h8*>(qf + 16 * st);
+            qlo[st] = *reinterpret_cast<const h8*>(qf + 16 * st + QPART);
+        }
+        qsc = s_qe[qg * 32 + n];
+        ek_lim = __builtin_amdgcn_readfirstlane(min(14 - s_eq, 128));
+        __syncthreads();
+    }
+
+    // reference max (log2 units, a whole number: it and the exponents add
+    // exactly), sum of p
+    int m = kNoMax;
+    float ls = 0.0f;
+    int e_acc = -112;                 // the sums' exponent E
+    v16f acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) acc[t][x] = 0.0f;
+
+    // sub-tile sub of tile i in buffer b; with CONV the loaded tile is split
+    // into the other buffer between the scores' matrix steps, and the one
+    // after it loaded
+    auto compute = [&](auto conv, int b, int sub, int i) __attribute__((always_inline)) {
+        constexpr bool CONV = decltype(conv)::value;
+        const int kb = i * C::KT + 32 * sub;
+        constexpr int PS = 4 * C::NP / NS;   // pairs split a step
+        const _Float16* kl = smem[b] + (32 * sub + n) * C::KP + 8 * h;
+        // (the small products in sums of their own: their roundings vanish,
+        // and the large ones meet half as many)
+        v16f s, sl;
+#pragma unroll
+        for (int x = 0; x < 16; ++x) s[x] = sl[x] = 0.0f;
+        h8 kph[2], kpl[2];
+        kph[0] = *reinterpret_cast<const h8*>(kl);
+        kpl[0] = *reinterpret_cast<const h8*>(kl + C::KPART);
+#pragma unroll
+        for (int st = 0; st < NS; ++st) {
+            // the next step's keys are read ahead; between the matrix steps
+            // run the split's instructions
+            if (st + 1 < NS) {
+                kph[(st + 1) & 1] = *reinterpret_cast<const h8*>(kl + 16 * (st + 1));
+                kpl[(st + 1) & 1] = *reinterpret_cast<const h8*>(kl + 16 * (st + 1) + C::KPART);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(kpl[st & 1], qhi[st], sl, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kph[st & 1], qhi[st], s, 0, 0, 0);
+            sl = __builtin_amdgcn_mfma_f32_32x32x16_f16(kph[st & 1], qlo[st], sl, 0, 0, 0);
+            if constexpr (CONV) {
+#pragma unroll
+                for (int x = 0; x < PS; ++x)
+                    convert(b ^ 1, (st * PS + x) >> 2, (st * PS + x) & 3);
+#pragma unroll
+                for (int x = 0; x < 3; ++x) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 2 * PS, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int x = 0; x < 16; ++x) s[x] += sl[x];
+        // elements 4j .. 4j+3: keys 8j + 4h + r
+        float c[4];
+        int evt = -1000;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            // (at least the smallest normal: -inf times c stays -inf)
+            c[j] = fmaxf(s_kf[b][(32 * sub + 8 * j) / C::KW] * qsc, 1.17549435e-38f);
+            evt = max(evt, __builtin_amdgcn_readfirstlane(s_ev[b][(4 * sub + j) / C::OW]));
+        }
+        if (KPOS || kb + 31 > min(qmin, n_kv - 1) || kb < klo_max) {
+            asm volatile("");   // (a branch: most steps skip this)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int i = 8 * j + r;   // key kb + i + 4h
+                    bool keep;
+                    if constexpr (KPOS) {
+                        const int32_t kp = s_kp[b][32 * sub + i + 4 * h];
+                        keep = kp <= qp && kp >= klo && kb + i + 4 * h < n_kv;
+                    } else {
+                        keep = i <= khi - kb - 4 * h && i >= klo - kb - 4 * h;
+                    }
+                    s[4 * j + r] = keep ? s[4 * j + r] : -INFINITY;
+                }
+        }
+        float tm = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float a = max3(s[4 * j], s[4 * j + 1], s[4 * j + 2]);
+            tm = max3(tm, a * c[j], s[4 * j + 3] * c[j]);
+        }
+        tm = fmaxf(tm, __shfl_xor(tm, 32));
+
+        // the sums follow the values' exponent (down only past 2^8, and not to
+        // a tile of zeros; sums that overflow for it are redone at the end)
+        // and the running max
+        const int e_new = evt > e_acc || (evt < e_acc - 8 && evt > -112) ? evt : e_acc;
+        // (the ceiling as a whole number; nothing kept, or a NaN: no max)
+        const int mt = tm > -INFINITY ? (int)ceilf(fminf(fmaxf(tm, -1e8f), 1e8f)) : kNoMax;
+        const int mn = max(m, mt);
+        const int da = max(m - mn, -1000) + e_acc - e_new;
+        const float alpha = da < -126 ? 0.0f : (da > 127 ? INFINITY : pow2i(da));
+        ls *= m - mn < -126 ? 0.0f : pow2i(m - mn);
+        m = mn;
+        e_acc = e_new;
+        const float msafe = m == kNoMax ? 0.0f : (float)m;   // p = 0 for a masked key
+        // p in units of 2^(ev - E), ev the octet's (keys 16k + 4h + r and 8
+        // more: elements 8k .. 8k+7); times 2^14 apart, so that the exponents
+        // that matter are near zero, where they round least
+        h8 phi[2], plo[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int fe = max(s_ev[b][(4 * sub + 2 * k + h) / C::OW] - e_acc, -54);
+            const float off = (float)fe - msafe;
+            float ps[4];
+            h2 hi[4], lo[4];
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                const float cj = c[2 * k + (x >> 1)];
+                const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * k + 2 * x], cj, off));
+                const float p1 =
+                    __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * k + 2 * x + 1], cj, off));
+                ps[x] = p0 + p1;
+                split_pair(p0 * 16384.0f, p1 * 16384.0f, hi[x], lo[x]);
+            }
+            ls += ((ps[0] + ps[1]) + (ps[2] + ps[3])) * pow2i(-fe);
+            phi[k] = __builtin_bit_cast(h8, make_uint4(h2_u32(hi[0]), h2_u32(hi[1]),
+                                                       h2_u32(hi[2]), h2_u32(hi[3])));
+            plo[k] = __builtin_bit_cast(h8, make_uint4(h2_u32(lo[0]), h2_u32(lo[1]),
+                                                       h2_u32(lo[2]), h2_u32(lo[3])));
+        }
+        const _Float16* vl = smem[b] + 2 * C::KPART + (sub * D + n) * C::VP;
+        // A step's keys are summed from zero and added to the sums once. During
+        // the matrix steps of 16 keys the next values are read, the last
+        // product of 32 dimensions is added to the sums, and (with CONV) a
+        // share of the next tile's loads is issued.
+        auto value = [&](int y) __attribute__((always_inline)) {   // y = 2t + k
+            return vl + 32 * (y >> 1) * C::VP + ((2 * (y & 1) + h) ^ ((2 * (y >> 1) + (n >> 4)) & 3)) * 8;
+        };
+        v16f o[2];
+        h8 vph[2], vpl[2];
+        vph[0] = *reinterpret_cast<const h8*>(value(0));
+        vpl[0] = *reinterpret_cast<const h8*>(value(0) + C::VPART);
+#pragma unroll
+        for (int y = 0; y < 2 * NT; ++y) {
+            const int t = y >> 1, k = y & 1, q = t & 1;
+            if (y + 1 < 2 * NT) {
+                vph[k ^ 1] = *reinterpret_cast<const h8*>(value(y + 1));
+                vpl[k ^ 1] = *reinterpret_cast<const h8*>(value(y + 1) + C::VPART);
+            }
+            if constexpr (CONV) {
+#pragma unroll
+                for (int x = 0; x < NL; ++x)
+                    if (x * 2 * NT / NL == y) load1(i + 2, x);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (k == 0) {
+#pragma unroll
+                for (int x = 0; x < 16; ++x) o[q][x] = 0.0f;
+            }
+            o[q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vpl[k], phi[k], o[q], 0, 0, 0);
+            o[q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vph[k], plo[k], o[q], 0, 0, 0);
+            o[q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vph[k], phi[k], o[q], 0, 0, 0);
+            if (t > 0) {
+#pragma unroll
+                for (int x = 8 * k; x < 8 * k + 8; ++x)
+                    acc[t - 1][x] = __builtin_fmaf(acc[t - 1][x], alpha, o[q ^ 1][x]);
+#pragma unroll
+                for (int x = 0; x < 3; ++x) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int x = 0; x < 16; ++x)
+            acc[NT - 1][x] = __builtin_fmaf(acc[NT - 1][x], alpha, o[(NT - 1) & 1][x]);
+    };
+
+    if (i_lo < i_hi) {
+        scales(0, i_lo);
+#pragma unroll
+        for (int x = 0; x < 4 * C::NP; ++x) convert(0, x >> 2, x & 3);
+        load(i_lo + 1);
+    }
+    __syncthreads();
+    for (int i = i_lo; i < i_hi; ++i) {
+        const int b = (i - i_lo) & 1;
+        // (past the last tile: zeros, into a buffer that nothing reads)
+        scales(b ^ 1, i + 1);
+        compute(std::true_type{}, b, gk, i);
+#pragma unroll
+        for (int sub = gk + C::GK; sub < C::SUBS; sub += C::GK)
+            compute(std::false_type{}, b, sub, i);
+        __syncthreads();
+    }
+
+    if (lane == 0) {
+        s_er[0][wave] = ev_lo;
+        s_er[1][wave] = ev_hi;
+    }
+    if constexpr (C::GK == 1) __syncthreads();
+    // back to natural units, the halves of a column added
+    ls += __shfl_xor(ls, 32);
+    const int back = e_acc - 28;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) acc[t][x] = ldexpf(acc[t][x], back);
+    if constexpr (C::GK == 2) {
+        // the second set of waves hands its sums to the first through LDS
+        float* xs = reinterpret_cast<float*>(&smem[0][0]) + qg * (64 * (16 * NT + 2)) + lane;
+        static_assert(4 * 64 * (16 * NT + 2) * 4 <= (int)sizeof(smem), "merge buffer");
+        if (gk == 1) {
+            xs[0] = (float)m;
+            xs[64] = ls;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int x = 0; x < 16; ++x) xs[64 * (2 + 16 * t + x)] = acc[t][x];
+        }
+        __syncthreads();
+        if (gk == 1) return;
+        const float m0 = (float)m, m1 = xs[0], l1 = xs[64];
+        const float mt = fmaxf(m0, m1);
+        const float w0 = __builtin_amdgcn_exp2f(m0 - mt), w1 = __builtin_amdgcn_exp2f(m1 - mt);
+        ls = ls * w0 + l1 * w1;
+        m = max(m, (int)m1);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int x = 0; x < 16; ++x)
+                acc[t][x] = acc[t][x] * w0 + xs[64 * (2 + 16 * t + x)] * w1;
+    }
+#pragma unroll
+    for (int x = 0; x < C::NW; ++x) {
+        ev_lo = min(ev_lo, s_er[0][x]);
+        ev_hi = max(ev_hi, s_er[1][x]);
+    }
+    // (scores past the clamp of m can leave no sum)
+    bool bad = ev_hi - ev_lo > 15 || s_bad != 0 || !(ls <= 3.4028235e38f) || (ls == 0.0f && m != kNoMax);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int x = 0; x < 16; ++x) bad = bad || !(fabsf(acc[t][x]) <= 3.4028235e38f);
+    if (__any(bad)) {
+        const int64_t u0 = tile * kSplitVecs + qg * 32;
+        attn_rows_plain<D>(p, u0, (int)max<int64_t>(0, min<int64_t>(32, n_vec - u0)), kh,
+                           KPOS ? 0 : i_lo * C::KT, KPOS ? n_kv : min(n_kv, i_hi * C::KT));
+        return;
+    }
+    if (qok) {
+        const float inv = 1.0f / fmaxf(ls, 1e-30f);
+        float* o = p.out + qrow * D + 4 * h;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                *reinterpret_cast<v4f*>(o + 32 * t + 8 * j) =
+                    v4f{acc[t][4 * j] * inv, acc[t][4 * j + 1] * inv, acc[t][4 * j + 2] * inv,
+                        acc[t][4 * j + 3] * inv};
+    }
+}

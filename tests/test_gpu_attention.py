@@ -15,7 +15,7 @@ import pytest
 from conftest import RTOL, bits_equal, golden, rel_to_scale
 from aero_amd import ops
 from aero_amd import transformer_native as TN
-from aero_amd.device import DeviceArray as DA
+from aero_amd.device import DeviceArray as DA, tune_set
 
 pytestmark = pytest.mark.gpu
 
@@ -398,3 +398,93 @@ def test_attention_random_shapes(hip, oracle, i, dt, T, H, HK, D, S, window):
         got = out.numpy()
         want = oracle.attention_tiled(q, kd, vd, scale, qpos=qpos, window=window or None)
     assert rel_to_scale(got, want) <= RTOL
+
+
+@pytest.fixture
+def split_always(hip):
+    """attn_split_kernel whatever the sizes."""
+    tune_set("attn_split", 2)
+    yield
+    tune_set("attn_split", None)
+
+
+@pytest.mark.parametrize("T,H,HK,D,S,window,kpos", [
+    (1, 4, 4, 64, 1, 0, False),          # one query, one key
+    (32, 4, 1, 64, 129, 0, False),       # 128 vectors exactly, one key past a tile
+    (33, 8, 2, 64, 127, 0, True),        # one token past a workgroup, shuffled keys
+    (65, 8, 2, 128, 65, 0, False),       # one key past the 64-key tile
+    (40, 6, 2, 128, 300, 33, False),     # 3 heads a kv head, a window across tiles
+    (70, 16, 2, 128, 190, 64, True),     # window and shuffled keys
+    (31, 4, 2, 256, 33, 0, False),       # one key past the 32-key tile
+    (90, 8, 4, 256, 200, 50, False),
+    (17, 16, 2, 256, 64, 0, True),
+])
+def test_split_vs_oracle(split_always, oracle, T, H, HK, D, S, window, kpos):
+    """The fp16-split kernel at the edges of its tiles; queries that keep no
+    key give exact zeros, and blocks of K / V of very different sizes meet."""
+    rng = np.random.default_rng(T + H + D + S + window)
+    q, k, v = rand_qkv(rng, T, H, HK, D, D, S)
+    k[S // 2:] *= 2.0 ** -20              # block exponents that move
+    v[S // 3:] *= 2.0 ** 12
+    qpos = np.arange(S - T, S, dtype=np.int32)
+    if T > 4:
+        qpos[0], qpos[1] = -3, S + 100
+    kp = rng.permutation(S).astype(np.int32) if kpos else None
+    print(f"split attention T={T} H={H} HK={HK} D={D} S={S} window={window}", flush=True)
+    scale = -1.0 / np.sqrt(D) if T == 40 else 1.0 / np.sqrt(D)
+    got = gpu_attention(q, k, v, scale, qpos=qpos, kpos=kp, window=window)
+    want = oracle.attention_tiled(q, k, v, scale, qpos=qpos, kpos=kp, window=window or None)
+    assert rel_to_scale(got, want) <= RTOL
+    if T > 4:
+        assert not got[0].any()
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan, 3.0e38])
+@pytest.mark.parametrize("where", ["q", "k", "v"])
+def test_split_non_finite(split_always, oracle, D, bad, where):
+    """A non-finite or huge operand touches the queries that keep it and no
+    other: those agree with the oracle's result without it; where the
+    fp32-step kernel gives the touched ones a finite row, so does this one."""
+    rng = np.random.default_rng(D)
+    T, H, HK, S = 70, 4, 2, 100
+    q, k, v = rand_qkv(rng, T, H, HK, D, D, S)
+    qpos = np.arange(S - T, S, dtype=np.int32)
+    scale = 1.0 / np.sqrt(D)
+    want = oracle.attention_tiled(q, k, v, scale, qpos=qpos)
+    {"q": q, "k": k, "v": v}[where][60, 1, 5] = bad
+    print(f"split attention D={D} {where} = {bad}", flush=True)
+    got = gpu_attention(q, k, v, scale, qpos=qpos)
+    touched = np.zeros((T, H), bool)
+    if where == "q":
+        touched[60, 1] = True
+    else:
+        touched[qpos >= 60, 2:] = True   # the heads of kv head 1
+    assert rel_to_scale(got[~touched], want[~touched]) <= RTOL
+    tune_set("attn_split", 0)
+    general = gpu_attention(q, k, v, scale, qpos=qpos)
+    tune_set("attn_split", 2)
+    for t, h in np.argwhere(touched):
+        if np.isfinite(general[t, h]).all():
+            assert rel_to_scale(got[t, h].astype(np.float64),
+                                general[t, h].astype(np.float64)) <= RTOL
+
+
+def test_split_rule_matches_general(hip):
+    """Calls on both sides of the rule's line agree with the fp32-step kernel,
+    a window, shuffled keys and cached prefixes among them."""
+    rng = np.random.default_rng(3)
+    for T, H, HK, D, S, window, kpos in [(256, 64, 8, 128, 256, 0, False),
+                                         (255, 32, 8, 64, 1300, 0, False),
+                                         (600, 14, 2, 64, 1700, 0, True),
+                                         (1024, 16, 2, 256, 1024, 300, False)]:
+        q, k, v = rand_qkv(rng, T, H, HK, D, D, S)
+        qpos = np.arange(S - T, S, dtype=np.int32)
+        kp = rng.permutation(S).astype(np.int32) if kpos else None
+        got = gpu_attention(q, k, v, 1.0 / np.sqrt(D), qpos=qpos, kpos=kp, window=window)
+        tune_set("attn_split", 0)
+        try:
+            want = gpu_attention(q, k, v, 1.0 / np.sqrt(D), qpos=qpos, kpos=kp, window=window)
+        finally:
+            tune_set("attn_split", None)
+        assert rel_to_scale(got, want) <= RTOL
