@@ -1,7 +1,8 @@
 // Quantised GEMM for many tokens on gfx950 (prefill): y[t, r] = sum_c W[r, c] * x[t, c]
 // with W in GGML blocks and x, y fp32 — the reference's matmul
 // (src/kernels.cpp:520-538) for token counts where re-reading W for every few
-// tokens (the GEMV kernels) would dominate.
+// tokens (the GEMV kernels) would dominate. Q8_0 runs gemm_q8_kernel (below);
+// the other types gemm_kernel:
 //
 // A workgroup (4 waves) computes a BM-row x BN-token tile of y. For each
 // BK-column chunk of the rows it dequantises its BM rows into LDS as fp32 —
@@ -14,7 +15,7 @@
 //
 // Weight staging: with W 16-byte aligned and rows a multiple of 16 bytes (8
 // for IQ4_XS) a thread dequantises one 32-value sub-block per chunk from
-// 16-byte loads (2-byte aligned Q8_0 / Q6_K blocks are shifted into place
+// 16-byte loads (2-byte aligned Q6_K blocks are shifted into place
 // with byte permutes); otherwise four values at a time from 2- and 4-byte
 // loads.
 //
@@ -106,31 +107,6 @@ template <> struct Sub32<AERO_DTYPE_Q5_K> {
     }
 };
 
-// Q8_0 (src/kernels.cpp:364-373): one block, 34 bytes at a 2-byte aligned
-// offset, from the 48 aligned bytes around it; y = d*q.
-template <> struct Sub32<AERO_DTYPE_Q8_0> {
-    uint4 c[3];
-    uint32_t ph;
-    __device__ __forceinline__ void load(const uint8_t* rowp, int c0) {
-        const uint32_t ob = (uint32_t)(c0 >> 5) * 34u;
-        ph = ob & 15u;
-        const uint8_t* b = rowp + (ob - ph);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) c[i] = ld128(b + 16 * i);
-    }
-    __device__ __forceinline__ void decode(float (&v)[32]) const {
-        uint32_t w[9];
-        shifted_words<9, 3>(c, ph, w);
-        const float d = half_bits_to_float(w[0] & 0xFFFFu);
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            const uint32_t q = __builtin_amdgcn_alignbyte(w[m + 1], w[m], 2);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[4 * m + e] = d * (float)(int8_t)((q >> (8 * e)) & 0xFFu);
-        }
-    }
-};
-
 // Q6_K (src/kernels.cpp:427-458): quarter kq of half h: nibble kq/2 of
 // ql[64h + 32(kq%2) + i], bits 2kq of qh[32h + i]; scale sc[8h + 2kq + i/16];
 // y = (d*sc)*(q-32). ql and qh from the 48 aligned bytes around each.
@@ -216,23 +192,19 @@ struct StageW<TYPE, true, BM, BK> {
     Sub32<TYPE> s[U];
     const uint8_t* rowp[U];
     int grp;
-    bool valid;
     __device__ __forceinline__ void init(const GemmParams& p, int64_t r0, int tid) {
         grp = tid % GR;
 #pragma unroll
         for (int u = 0; u < U; ++u)
             rowp[u] = p.w + min(r0 + (tid + 256 * u) / GR, p.n_rows - 1) * p.rb;
     }
-    __device__ __forceinline__ void load(const GemmParams& p, int kc) {
+    __device__ __forceinline__ void load(const GemmParams&, int kc) {
         const int c = kc * BK + 32 * grp;
-        valid = c < p.n_cols;  // n_cols is a multiple of 32
-        const int cc = min(c, p.n_cols - 32);
 #pragma unroll
-        for (int u = 0; u < U; ++u) s[u].load(rowp[u], cc);
+        for (int u = 0; u < U; ++u) s[u].load(rowp[u], c);
     }
     __device__ __forceinline__ void store(float* As, int tid) const {
         constexpr int RowF = BK + 4;
-        const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             float v[32];
@@ -240,14 +212,10 @@ struct StageW<TYPE, true, BM, BK> {
             float* row = As + ((tid + 256 * u) / GR) * RowF + 8 * grp;
 #pragma unroll
             for (int kk = 0; kk < 4; ++kk) {
-                // past n_cols (the last chunk of a Q8_0 row whose length is
-                // not a multiple of 128): zeros, replacing the values of the
-                // clamped block (a multiply by zero would keep inf / nan)
-                float4 a = make_float4(v[kk], v[kk + 4], v[kk + 8], v[kk + 12]);
-                float4 b = make_float4(v[kk + 16], v[kk + 20], v[kk + 24], v[kk + 28]);
-                if (!valid) a = b = z;
-                *reinterpret_cast<float4*>(row + kk * (BK / 4)) = a;
-                *reinterpret_cast<float4*>(row + kk * (BK / 4) + 4) = b;
+                *reinterpret_cast<float4*>(row + kk * (BK / 4)) =
+                    make_float4(v[kk], v[kk + 4], v[kk + 8], v[kk + 12]);
+                *reinterpret_cast<float4*>(row + kk * (BK / 4) + 4) =
+                    make_float4(v[kk + 16], v[kk + 20], v[kk + 24], v[kk + 28]);
             }
         }
     }
@@ -262,17 +230,14 @@ struct StageW<TYPE, false, BM, BK> {
     Raw raw[U][4];
     const uint8_t* rowp[U];
     int grp, cc;
-    bool valid;
     __device__ __forceinline__ void init(const GemmParams& p, int64_t r0, int tid) {
         grp = tid % GR;
 #pragma unroll
         for (int u = 0; u < U; ++u)
             rowp[u] = p.w + min(r0 + (tid + 256 * u) / GR, p.n_rows - 1) * p.rb;
     }
-    __device__ __forceinline__ void load(const GemmParams& p, int kc) {
-        const int c = kc * BK + 16 * grp;
-        valid = c < p.n_cols;
-        cc = min(c, p.n_cols - 16);
+    __device__ __forceinline__ void load(const GemmParams&, int kc) {
+        cc = kc * BK + 16 * grp;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int cq = cc + 4 * q;
@@ -284,14 +249,12 @@ struct StageW<TYPE, false, BM, BK> {
     }
     __device__ __forceinline__ void store(float* As, int tid) const {
         constexpr int RowF = BK + 4;
-        const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             float4 w4[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const float4 dq = decode(raw[u][q], ((cc + 4 * q) % QT<TYPE>::BV) / 4);
-                w4[q] = valid ? dq : z;  // decode unconditional: a select, not a branch
+                w4[q] = decode(raw[u][q], ((cc + 4 * q) % QT<TYPE>::BV) / 4);
             }
             float* row = As + ((tid + 256 * u) / GR) * RowF + 4 * grp;
             *reinterpret_cast<float4*>(row + 0 * BK / 4) = make_float4(w4[0].x, w4[1].x, w4[2].x, w4[3].x);
@@ -427,19 +390,244 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams p) {
         }
 }
 
+// ------------------------------------------------------- Q8_0, bf16 parts
+// y[t, r] = sum_b d_b sum_c q_c x_c over Q8_0 blocks b of 32: a matrix step of
+// v_mfma_f32_16x16x32_bf16 covers one block of 16 rows and 16 tokens. int8
+// codes are exact in bf16, and x is the exact sum of three bf16 parts (its 24
+// bits cut after 8 and 16), so every product is exact; a block's three steps,
+// the smallest part first, are summed in fp32 from zero and added to the
+// row's sum times d, one rounding a block. (D holds tokens 4(l/16) + v of row
+// l%16: d is lane-local. Lane l supplies columns 8(l/16) .. +7 of token l%16
+// and of row l%16, loaded as they lie.)
+//
+// The four waves of a workgroup own the same NT x 16 rows and MT x 16 tokens
+// and take every fourth block; their sums meet in LDS once at the end, so
+// the loop has no barrier and no LDS traffic, and short rows (896 columns: 28
+// blocks) still keep four waves busy. A part of x costs vector instructions
+// per row tile instead (about as long as the matrix steps at NT = 2).
+// Measured on MI355X against the fp32 matrix steps of gemm_kernel (2.7 times
+// the matrix time, 128-column chunks between barriers): see launch_q8.
+typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
+typedef uint32_t u3w __attribute__((ext_vector_type(3), aligned(4)));
+
+// 8 int8 codes (two dwords) as bf16: each byte offset by 128, converted and
+// shifted back (exact), the upper halves of the floats packed
+__device__ __forceinline__ bf8v q8_bf16(uint32_t w0, uint32_t w1) {
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t u = (i ? w1 : w0) ^ 0x80808080u;
+        const float f0 = (float)(u & 255u) - 128.0f, f1 = (float)((u >> 8) & 255u) - 128.0f;
+        const float f2 = (float)((u >> 16) & 255u) - 128.0f, f3 = (float)(u >> 24) - 128.0f;
+        o[2 * i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f1),
+                                         __builtin_bit_cast(uint32_t, f0), 0x07060302u);
+        o[2 * i + 1] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f3),
+                                             __builtin_bit_cast(uint32_t, f2), 0x07060302u);
+    }
+    return __builtin_bit_cast(bf8v, make_uint4(o[0], o[1], o[2], o[3]));
+}
+
+// 8 floats as three bf16 parts (part 0 the largest); an infinity keeps part 0
+__device__ __forceinline__ void bf16_parts(const float (&x)[8], bf8v (&p)[3]) {
+    float r[3][8];
+    float big = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float h = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x[i]) & 0xFFFF0000u);
+        r[0][i] = h;
+        r[1][i] = x[i] - h;
+        const float m =
+            __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r[1][i]) & 0xFFFF0000u);
+        r[2][i] = r[1][i] - m;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i += 2)
+        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(big) : "v"(x[i]), "v"(x[i + 1]));
+    if (__any(big > 3.4028235e38f)) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (fabsf(x[i]) > 3.4028235e38f) r[1][i] = r[2][i] = 0.0f;
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        uint32_t o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            o[i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, r[k][2 * i + 1]),
+                                         __builtin_bit_cast(uint32_t, r[k][2 * i]), 0x07060302u);
+        p[k] = __builtin_bit_cast(bf8v, make_uint4(o[0], o[1], o[2], o[3]));
+    }
+}
+
+template <int MT, int NT, int KW>
+__global__ __launch_bounds__(64 * KW) void gemm_q8_kernel(GemmParams p) {
+    __shared__ v4f sums[KW][MT * NT][64];
+    const int l = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = l & 15, g = l >> 4;
+    const int64_t r0 = (int64_t)blockIdx.x * (16 * NT);
+    const int t0 = blockIdx.y * (16 * MT);
+    const int nb = p.n_cols / 32;
+
+    // lane's rows and tokens (clamped: the copies are not stored)
+    const uint8_t* wp[NT];
+    const float* xp[MT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+        wp[j] = p.w + min(r0 + 16 * j + c, p.n_rows - 1) * p.rb;
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+        xp[m] = p.x + (int64_t)min(t0 + 16 * m + c, p.n_tok - 1) * p.x_stride + 8 * g;
+
+    float4 xa[MT][2];
+    u3w wq[NT];
+    uint32_t wd[NT];
+    // the codes lie 2 bytes off a dword in every other block (and row, where
+    // their number is odd): the dwords around them, shifted into place; the
+    // last dword holds at least two of the codes
+    auto load = [&](int b) __attribute__((always_inline)) {
+        b = min(b, nb - 1);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            xa[m][0] = *reinterpret_cast<const float4*>(xp[m] + 32 * b);
+            xa[m][1] = *reinterpret_cast<const float4*>(xp[m] + 32 * b + 4);
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const uint8_t* e = wp[j] + (int64_t)34 * b;
+            const uintptr_t a = reinterpret_cast<uintptr_t>(e + 2 + 8 * g);
+            // (aligned: dwords 0 and 1, and dword 1 again; else 0, 1 and 2)
+            const uint32_t* d = reinterpret_cast<const uint32_t*>(a & ~uintptr_t(3));
+            wq[j][0] = d[0];
+            wq[j][1] = d[1];
+            wq[j][2] = d[(a & 2) ? 2 : 1];
+            wd[j] = *reinterpret_cast<const uint16_t*>(e);
+        }
+    };
+
+    v4f acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[m][j] = v4f{0.f, 0.f, 0.f, 0.f};
+
+    load(wave);
+    for (int b = wave; b < nb; b += KW) {
+        bf8v wb[NT];
+        float d[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const uint32_t sh = (uint32_t)(reinterpret_cast<uintptr_t>(wp[j] + (int64_t)34 * b + 2) & 2);
+            wb[j] = q8_bf16(__builtin_amdgcn_alignbyte(wq[j][1], wq[j][0], sh),
+                            __builtin_amdgcn_alignbyte(wq[j][2], wq[j][1], sh));
+            d[j] = half_bits_to_float(wd[j]);
+        }
+        bf8v xb[MT][3];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const float x[8] = {xa[m][0].x, xa[m][0].y, xa[m][0].z, xa[m][0].w,
+                                xa[m][1].x, xa[m][1].y, xa[m][1].z, xa[m][1].w};
+            bf16_parts(x, xb[m]);
+        }
+        load(b + KW);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                v4f part = {0.f, 0.f, 0.f, 0.f};
+                part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xb[m][2], wb[j], part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xb[m][1], wb[j], part, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xb[m][0], wb[j], part, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    acc[m][j][v] = __builtin_fmaf(part[v], d[j], acc[m][j][v]);
+            }
+    }
+
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) sums[wave][m * NT + j][l] = acc[m][j];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MT * NT; i += KW) {
+        if (i + wave >= MT * NT) break;
+        const int m = (i + wave) / NT, j = (i + wave) % NT;
+        v4f y = sums[0][i + wave][l];
+#pragma unroll
+        for (int k = 1; k < KW; ++k) y += sums[k][i + wave][l];
+        const int64_t row = r0 + 16 * j + c;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int tok = t0 + 16 * m + 4 * g + v;
+            if (row < p.n_rows && tok < p.n_tok) p.y[(int64_t)tok * p.y_stride + row] = y[v];
+        }
+    }
+}
+
 using GemmKernel = void (*)(GemmParams);
 
 template <bool FAST>
 GemmKernel pick_gemm(int dtype) {
     constexpr int BM = 64, BN = 64, BK = 128;
     switch (dtype) {
-    case AERO_DTYPE_Q8_0: return gemm_kernel<AERO_DTYPE_Q8_0, FAST, BM, BN, BK>;
     case AERO_DTYPE_Q4_K: return gemm_kernel<AERO_DTYPE_Q4_K, FAST, BM, BN, BK>;
     case AERO_DTYPE_Q5_K: return gemm_kernel<AERO_DTYPE_Q5_K, FAST, BM, BN, BK>;
     case AERO_DTYPE_Q6_K: return gemm_kernel<AERO_DTYPE_Q6_K, FAST, BM, BN, BK>;
     case AERO_DTYPE_IQ4_XS: return gemm_kernel<AERO_DTYPE_IQ4_XS, FAST, BM, BN, BK>;
     default: return nullptr;
     }
+}
+
+}  // namespace
+
+namespace {
+
+// A workgroup tile of gemm_q8_kernel and its cost a block step with one
+// workgroup a CU (measured on MI355X, us for eight waves taking a block each,
+// 896 x 4864).
+struct Q8Tile {
+    int mt, nt;
+    double cost;
+    void (*k)(GemmParams);
+};
+constexpr int kQ8Waves = 8;
+const Q8Tile kQ8Tiles[] = {
+    {1, 1, 0.65, gemm_q8_kernel<1, 1, kQ8Waves>}, {2, 1, 1.05, gemm_q8_kernel<2, 1, kQ8Waves>},
+    {1, 2, 1.15, gemm_q8_kernel<1, 2, kQ8Waves>}, {2, 2, 1.50, gemm_q8_kernel<2, 2, kQ8Waves>},
+    {4, 2, 2.35, gemm_q8_kernel<4, 2, kQ8Waves>}, {2, 4, 2.50, gemm_q8_kernel<2, 4, kQ8Waves>},
+    {4, 4, 3.30, gemm_q8_kernel<4, 4, kQ8Waves>},
+};
+
+// The tile whose rounds of one workgroup a CU cost least. Measured on MI355X,
+// fp32-step GEMM (GEMV below 32 tokens) / this in us: 4864 x 896 at 8 tokens
+// 13.8 / 6.2, 32 30.6 / 8.1, 77 31.8 / 12.1, 512 75.8 / 41.3; 896 x 4864 at
+// 77 116 / 24.7; 4096 x 4096 at 512 171 / 151; 14336 x 4096 at 64 100.5 /
+// 76.6, 512 577 / 522. Error against float64 at 896 columns 5.3e-7 -> 7.6e-8.
+// (AERO_HIP_TUNE gemm_q8_tile=N takes entry N - 1 instead.)
+bool launch_q8(const GemmParams& p, hipStream_t s) {
+    const int64_t cus = cu_count();
+    auto wgs = [&](const Q8Tile& t) {
+        return (p.n_rows + 16 * t.nt - 1) / (16 * t.nt) *
+               (((int64_t)p.n_tok + 16 * t.mt - 1) / (16 * t.mt));
+    };
+    const Q8Tile* best = nullptr;
+    double least = 0.0;
+    for (const Q8Tile& t : kQ8Tiles) {
+        if (((int64_t)p.n_tok + 16 * t.mt - 1) / (16 * t.mt) > 65535) continue;
+        const double c = (double)((wgs(t) + cus - 1) / cus) * t.cost;
+        if (best == nullptr || c < least) {
+            best = &t;
+            least = c;
+        }
+    }
+    const int fixed = tune("gemm_q8_tile", 0);
+    if (fixed >= 1 && fixed <= (int)(sizeof(kQ8Tiles) / sizeof(kQ8Tiles[0])))
+        best = &kQ8Tiles[fixed - 1];
+    const int64_t rt = (p.n_rows + 16 * best->nt - 1) / (16 * best->nt);
+    const int64_t tt = ((int64_t)p.n_tok + 16 * best->mt - 1) / (16 * best->mt);
+    return launch("gemm_q8_kernel", best->k, dim3((unsigned)rt, (unsigned)tt),
+                  dim3(64 * kQ8Waves), 0, s, p);
 }
 
 }  // namespace
@@ -453,13 +641,15 @@ bool gemm_dev(int dtype, const uint8_t* w, const float* x, float* y, int64_t n_r
     const bool fast = dtype == AERO_DTYPE_IQ4_XS
                           ? (reinterpret_cast<uintptr_t>(w) & 7u) == 0 && rb % 8 == 0
                           : aligned16(w) && rb % 16 == 0;
+    const GemmParams p{w, x, y, n_rows, (int)n_cols, rb, (int)n_tok, n_cols, n_rows};
+    if (dtype == AERO_DTYPE_Q8_0 && row_tiles <= 0x1fffffff && tok_tiles <= 65535)
+        return launch_q8(p, s);
     GemmKernel k = (fast && tune("gemm_fast", 1)) ? pick_gemm<true>(dtype) : pick_gemm<false>(dtype);
     if (k == nullptr || row_tiles > 0x7fffffff || tok_tiles > 65535 || n_cols % 32 != 0) {
         set_error("matmul: no GEMM for dtype %d at %lld x %lld, %lld tokens", dtype,
                   (long long)n_rows, (long long)n_cols, (long long)n_tok);
         return false;
     }
-    GemmParams p{w, x, y, n_rows, (int)n_cols, rb, (int)n_tok, n_cols, n_rows};
     return launch("gemm_kernel", k, dim3((unsigned)row_tiles, (unsigned)tok_tiles), dim3(256), 0,
                   s, p);
 }

@@ -1871,6 +1871,14 @@ bool split_gemm_dev(int dtype, const uint8_t* w, const float* x, float* y, int64
         !aligned16(ws) || !tune("gemm16", 1))
         return true;
     if (!split_room_ok(n_rows, n_cols, n_tok, ws_bytes - need)) return true;
+    // Q8_0 rows whose super-blocks do not divide (4864 columns: 19) would run
+    // unsplit on a part of the chip: gemm_q8_kernel, whose waves share the
+    // columns, takes them. Measured on MI355X, 896 x 4864, this / that in us:
+    // 16 tokens 45.0 / 16.9, 77 47.6 / 25.5, 256 50.4 / 35.1, 512 52.6 / 51.6.
+    const int64_t base_wgs = (n_rows + 127) / 128 * (pad_tokens(n_tok) / kTokTile);
+    if (dtype == AERO_DTYPE_Q8_0 && base_wgs < 128 && tune("gemm16_nt", 2) == 2 &&
+        pick_ksplit(base_wgs, (int)(n_cols / 256), n_tok * n_rows * 4, ws_bytes - need) == 1)
+        return true;
     SplitJob j{dtype, x, nullptr, nullptr, nullptr, -1, 0.f, 1, &w, nullptr, 0, &n_rows, &y,
                n_cols, rb, n_tok, ws, {}, ws_bytes};
     if (!split_run(j, s)) return false;

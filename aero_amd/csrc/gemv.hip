@@ -1650,14 +1650,22 @@ bool gemv_dev(int dtype, const uint8_t* w, int64_t w_bytes, const float* x, floa
     // several tokens: the matrix-core GEMMs. The split-x fp16 one when a
     // workspace is given and the type has it (from 5-16 tokens by the
     // matrix size, split_tokens_ok), else the fp32 one from 32 tokens (W
-    // once per 64).
+    // once per 64), or Q8_0's bf16 one from 5 where the GEMV takes rows of up
+    // to half a step or more than one, from 13 where it takes 4 tokens a
+    // launch of one-step rows. Measured on MI355X, GEMV / GEMM in us: 4864 x
+    // 896 at 4 tokens 7.2 / 6.3, 8 13.8 / 6.2; 896 x 4864 at 4 12.8 / 13.9, 5
+    // 17.3 / 13.9; 512 x 2048 at 5 9.0 / 9.0, 8 11.7 / 9.7; 1024 x 4096 at 8
+    // 11.9 / 17.2, 12 17.5 / 18.3; 14336 x 4096 at 5 39.9 / 52.5.
     if (ws != nullptr && n_tok <= (int64_t)1 << 30 && split_tokens_ok(n_tok, n_rows, n_cols)) {
         bool ran = false;
         if (!split_gemm_dev(dtype, w, x, y, n_rows, n_cols, rb, n_tok, ws, ws_bytes, s, &ran))
             return false;
         if (ran) return true;
     }
-    if (n_tok >= tune("gemm_min_tokens", 32) && n_tok <= (int64_t)1 << 30)
+    const int min_tok = dtype != AERO_DTYPE_Q8_0 ? 32
+                        : 2 * n_cols <= kStepCols || n_cols > kStepCols ? 5 : 13;
+    if (n_tok >= tune("gemm_min_tokens", min_tok) &&
+        n_tok <= (int64_t)1 << 30)
         return gemm_dev(dtype, w, x, y, n_rows, n_cols, rb, n_tok, s);
     if (lanes64_ok(dtype, w, rb, n_rows, w_bytes) && tune("gemv_lanes64", 1)) {
         const bool pipe = n_cols > kStepCols;

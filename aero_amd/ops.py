@@ -258,7 +258,8 @@ def matvec(dtype: int, w: DeviceArray, x: DeviceArray, y: DeviceArray, n_rows: i
     blocks (Q8_0, Q4_K, Q5_K, Q6_K, IQ4_XS), x [n_tok, n_cols], y [n_tok, n_rows].
     From 5-16 tokens (by matrix size), Q4_K, Q5_K, Q8_0, Q6_K (rows of 2048k
     columns) and IQ4_XS (512k) run the split-x fp16 matrix-core GEMM with a
-    cached workspace (split=False: the fp32 matrix-core GEMM)."""
+    cached workspace (split=False: the GEMMs that need none, Q8_0 on bf16
+    matrix steps, the others on fp32 ones)."""
     if dtype not in _BLOCK or _BLOCK[dtype][0] == 1:
         raise ValueError(f"dtype {dtype} has no quantised GEMV")
     bv, bb = _BLOCK[dtype]

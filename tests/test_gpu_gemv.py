@@ -12,7 +12,7 @@ import pytest
 from conftest import RTOL, golden, rel_to_scale
 from aero_amd import native, ops
 from aero_amd import workloads as W
-from aero_amd.device import DeviceArray as DA
+from aero_amd.device import DeviceArray as DA, tune_set
 
 pytestmark = pytest.mark.gpu
 
@@ -184,3 +184,69 @@ def test_norm_matvec_half_wave_odd_rows(hip, oracle, n_tok):
     h = oracle.rmsnorm_rows(x, nw, 1e-5)
     for w, r, y in zip(ws, rows, ys):
         assert rel_to_scale(y.numpy(), oracle.matmul(t, w, h, r)) <= RTOL
+
+
+@pytest.mark.parametrize("tile", range(1, 8))
+@pytest.mark.parametrize("n_rows,n_cols,n_tok", [
+    (1, 32, 5),        # one block a row: seven of the eight waves have none
+    (17, 96, 17),      # an odd block count: rows start 2 bytes off a dword
+    (65, 896, 64),     # one row past four tiles, whole token tiles
+    (130, 4864, 65),   # one token past four tiles
+    (33, 544, 6),
+])
+def test_gemm_q8_tiles(hip, oracle, n_rows, n_cols, n_tok, tile):
+    """gemm_q8_kernel's tiles at their edges (split=False: no workspace)."""
+    rng = np.random.default_rng(n_rows + n_cols + n_tok)
+    w = W.make_table(W.Q8_0, n_rows * n_cols // 32, rng)
+    X = rng.standard_normal((n_tok, n_cols)).astype(np.float32)
+    X *= np.exp2(rng.integers(-30, 30, (n_tok, 1))).astype(np.float32)
+    y = DA.empty((n_tok, n_rows))
+    print(f"gemm_q8 tile={tile} rows={n_rows} cols={n_cols} tokens={n_tok}", flush=True)
+    tune_set("gemm_q8_tile", tile)
+    try:
+        ops.matvec(W.Q8_0, DA.from_numpy(w), DA.from_numpy(X), y, n_rows, n_cols, n_tok,
+                   split=False)
+    finally:
+        tune_set("gemm_q8_tile", None)
+    want = oracle.matmul(W.Q8_0, w, X, n_rows)
+    for t in range(n_tok):                # a token's scale is its own
+        assert rel_to_scale(y.numpy()[t], want[t]) <= RTOL
+
+
+def test_gemm_q8_non_finite(hip, oracle):
+    """An infinity or NaN in x reaches its token only, an infinity with the
+    sign that the exact product has."""
+    rng = np.random.default_rng(9)
+    n_rows, n_cols, n_tok = 40, 896, 20
+    w = W.make_table(W.Q8_0, n_rows * n_cols // 32, rng)
+    X = rng.standard_normal((n_tok, n_cols)).astype(np.float32)
+    clean = oracle.matmul(W.Q8_0, w, X, n_rows)
+    X[3, 100], X[7, 5], X[11, 800] = np.inf, -np.inf, np.nan
+    y = DA.empty((n_tok, n_rows))
+    ops.matvec(W.Q8_0, DA.from_numpy(w), DA.from_numpy(X), y, n_rows, n_cols, n_tok, split=False)
+    got = y.numpy()
+    with np.errstate(all="ignore"):
+        want = oracle.matmul(W.Q8_0, w, X, n_rows)
+    keep = [t for t in range(n_tok) if t not in (3, 7, 11)]
+    assert rel_to_scale(got[keep], clean[keep]) <= RTOL
+    assert np.isnan(got[11]).all()
+    for t in (3, 7):
+        assert np.array_equal(np.isnan(got[t]), np.isnan(want[t]))
+        assert np.array_equal(np.sign(got[t]), np.sign(want[t]), equal_nan=True)
+
+
+@pytest.mark.parametrize("n_rows,n_cols,n_tok", [(896, 4864, 16), (896, 4864, 100),
+                                                 (1024, 4096, 12), (1024, 4096, 13),
+                                                 (512, 2048, 5), (130, 5120, 5), (130, 2304, 5)])
+def test_q8_routes_agree(hip, oracle, n_rows, n_cols, n_tok):
+    """Q8_0 calls on both sides of the lines between GEMV, gemm_q8_kernel and
+    the split GEMM, with and without the workspace."""
+    rng = np.random.default_rng(n_rows + n_cols + n_tok)
+    w = W.make_table(W.Q8_0, n_rows * n_cols // 32, rng)
+    X = rng.standard_normal((n_tok, n_cols)).astype(np.float32)
+    want = oracle.matmul(W.Q8_0, w, X, n_rows)
+    dw, dx, y = DA.from_numpy(w), DA.from_numpy(X), DA.empty((n_tok, n_rows))
+    for split in (True, False):
+        ops.matvec(W.Q8_0, dw, dx, y, n_rows, n_cols, n_tok, split=split)
+        assert rel_to_scale(y.numpy(), want) <= RTOL
+
