@@ -1403,11 +1403,23 @@ struct ReduceArgs {
     float* y[kMaxMats];
     int64_t n_rows[kMaxMats];
     int64_t roff[kMaxMats + 1];
+    // RoPE on the outputs of matrices 0 .. rope_mats-1 (SplitParams)
+    int rope_mats;
+    int rope_D;
+    int rope_rot;
+    int rope_mode;
+    const int32_t* pos;
+    const float* rinv;
 };
 
-template <int EPI>
+// With ROPE (plain form, heads of rope_D outputs that a workgroup's 256 hold
+// whole) an output meets its partner in LDS and is stored rotated: the pass
+// over q and k that a column-split call would run otherwise (16 tokens of
+// Llama-3-8B's add + norm + q, k, v + RoPE on MI355X: 24.0 -> 21.7 us).
+template <int EPI, bool ROPE = false>
 __global__ __launch_bounds__(256) void split_reduce_kernel(ReduceArgs a) {
     constexpr bool GU = EPI != kEpiPlain;
+    static_assert(!ROPE || !GU, "RoPE on plain products");
     const int tid = threadIdx.x;
     const int tok = blockIdx.y;
     __shared__ float tinv;
@@ -1434,7 +1446,7 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(ReduceArgs a) {
     }
     __syncthreads();
     const float inv = tinv;
-    if (o >= n_out) return;
+    if (!ROPE && o >= n_out) return;
     float gv = 0.f, uv = 0.f;
 #pragma unroll
     for (int z = 0; z < kMaxSplits; ++z) {
@@ -1453,6 +1465,25 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(ReduceArgs a) {
         int m = 0;
 #pragma unroll
         for (int i = 1; i < kMaxMats; ++i) m += (i < a.n_mat && o >= a.roff[i]);
+        if constexpr (ROPE) {
+            __shared__ float head[256];
+            head[tid] = gv;
+            __syncthreads();
+            const int q = (int)((o - a.roff[m]) % a.rope_D);
+            if (m < a.rope_mats && o < n_out && q < a.rope_rot) {
+                // x0 c - x1 s, x0 s + x1 c (src/transformer.cpp:77-93)
+                const bool neox = a.rope_mode == AERO_ROPE_NEOX;
+                const int half = a.rope_rot / 2;
+                const bool second = neox ? q >= half : (q & 1) != 0;
+                const int qi = neox ? (second ? q - half : q) : q >> 1;
+                const int step = neox ? half : 1;
+                const float other = head[second ? tid - step : tid + step];
+                float sn, c;
+                sincosf((float)a.pos[tok] * a.rinv[qi], &sn, &c);
+                gv = second ? other * sn + gv * c : gv * c - other * sn;
+            }
+            if (o >= n_out) return;
+        }
         a.y[m][(int64_t)tok * a.n_rows[m] + (o - a.roff[m])] = gv;
     }
 }
@@ -1645,6 +1676,19 @@ bool split_rope_ok(const SplitJob& j, int rows_wg, int ks, int mt) {
     return true;
 }
 
+// Whether the reduction of a column-split call applies j.rope: no per-head
+// norm, and heads that its 256-output workgroups hold whole.
+bool reduce_rope_ok(const SplitJob& j) {
+    const RopeFold& r = j.rope;
+    if (r.mats < 1 || j.w_up != nullptr || r.mats > j.n_mat || r.qk_norm() || r.pos == nullptr ||
+        r.inv == nullptr || r.D < 2 || 256 % r.D || r.rot() < 2 || r.rot() > r.D ||
+        r.rot() % 2 || (r.mode != AERO_ROPE_NEOX && r.mode != AERO_ROPE_INTERLEAVED))
+        return false;
+    for (int m = 0; m < r.mats; ++m)
+        if (j.n_rows[m] % r.D) return false;
+    return true;
+}
+
 bool split_run(const SplitJob& j, hipStream_t s, bool* rope_done = nullptr) {
     if (rope_done != nullptr) *rope_done = false;
     const int64_t tp = pad_tokens(j.n_tok);
@@ -1806,6 +1850,17 @@ bool split_run(const SplitJob& j, hipStream_t s, bool* rope_done = nullptr) {
     const dim3 rg((unsigned)((n_out + 255) / 256), (unsigned)j.n_tok);
     switch (epi) {
     case kEpiPlain:
+        if (reduce_rope_ok(j)) {
+            ra.rope_mats = j.rope.mats;
+            ra.rope_D = j.rope.D;
+            ra.rope_rot = j.rope.rot();
+            ra.rope_mode = j.rope.mode;
+            ra.pos = j.rope.pos;
+            ra.rinv = j.rope.inv;
+            if (rope_done != nullptr) *rope_done = true;
+            return launch("split_reduce_kernel", split_reduce_kernel<kEpiPlain, true>, rg,
+                          dim3(256), 0, s, ra);
+        }
         return launch("split_reduce_kernel", split_reduce_kernel<kEpiPlain>, rg, dim3(256), 0, s, ra);
     case AERO_ACT_SILU:
         return launch("split_reduce_kernel", split_reduce_kernel<AERO_ACT_SILU>, rg, dim3(256), 0, s,

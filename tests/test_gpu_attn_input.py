@@ -149,6 +149,26 @@ def test_attn_input_64_token_workgroups(hip, oracle, case):
     assert n == 2, n
 
 
+@pytest.mark.parametrize("wt,T,N,D,heads,n_rot,mode,qk,src", [
+    (W.Q4_K, 16, 2048, 128, (4, 1, 1), 128, NEOX, False, "resid"),
+    (W.Q4_K, 17, 1024, 64, (3, 1, 1), 32, INTER, False, "emb"),     # 320 outputs
+    (W.Q8_0, 31, 2048, 256, (2, 1, 1), 64, NEOX, False, "x"),       # a head a workgroup
+    (W.Q5_K, 16, 1024, 32, (5, 2, 2), 32, INTER, False, "resid"),
+    (W.Q4_K, 16, 2048, 128, (4, 1, 1), 128, NEOX, True, "resid"),   # a head norm: its own pass
+])
+def test_attn_input_column_split(hip, oracle, wt, T, N, D, heads, n_rot, mode, qk, src):
+    """Few tokens split the columns: the reduction over the partials rotates
+    q and k (no head norm), against the oracle."""
+    dmats, rows, kw_args, ys = run_case(oracle, wt, W.Q4_K, T, N, D, heads, n_rot, mode, qk,
+                                        False, src, seed=T + N + D)
+    plan = Plan()
+    with plan:
+        ops.attn_input(wt, dmats, [DA.empty(y.shape) for y in ys], rows, N, T, **kw_args)
+    n = len(plan)
+    plan.destroy()
+    assert n == (4 if qk else 3), n    # pre-pass, GEMM, reduction (, the per-head pass)
+
+
 def test_attn_input_llama3_8b_512_tokens(hip, oracle):
     """The Llama-3-8B block's attention input at 512 tokens (hidden 4096,
     32/8 heads of 128, Q4_K weights and table): two launches, checked on a
