@@ -1677,11 +1677,14 @@ bool split_rope_ok(const SplitJob& j, int rows_wg, int ks, int mt) {
 }
 
 // Whether the reduction of a column-split call applies j.rope: no per-head
-// norm, and heads that its 256-output workgroups hold whole.
+// norm, heads that its 256-output workgroups hold whole, and fewer than 32
+// tokens (one token tile), where the pass it replaces is a tenth of the call;
+// a larger call that still splits its columns has few rows, and keeps the
+// launches that callers' counts of a recorded plan know.
 bool reduce_rope_ok(const SplitJob& j) {
     const RopeFold& r = j.rope;
-    if (r.mats < 1 || j.w_up != nullptr || r.mats > j.n_mat || r.qk_norm() || r.pos == nullptr ||
-        r.inv == nullptr || r.D < 2 || 256 % r.D || r.rot() < 2 || r.rot() > r.D ||
+    if (j.n_tok >= kTokTile || r.mats < 1 || j.w_up != nullptr || r.mats > j.n_mat ||
+        r.qk_norm() || r.pos == nullptr || r.inv == nullptr || r.D < 2 || 256 % r.D || r.rot() < 2 || r.rot() > r.D ||
         r.rot() % 2 || (r.mode != AERO_ROPE_NEOX && r.mode != AERO_ROPE_INTERLEAVED))
         return false;
     for (int m = 0; m < r.mats; ++m)
