@@ -43,8 +43,8 @@
 // and a step takes about 7500: two waves a SIMD (all 256 registers each) do
 // not overlap them fully. Against attn_mfma_kernel, whose fp32 steps run at a
 // sixteenth of the fp16 rate, on MI355X, 2048 causal tokens: 32 / 8 heads of
-// dim 128 463 -> 150 us (229 TFLOP/s by the useful products), of dim 64
-// 256 -> 85 us, 8 / 4 heads of dim 256 in a window of 1024 222 -> 146 us.
+// dim 128 454 -> 149 us (231 TFLOP/s by the useful products), of dim 64
+// 252 -> 86 us, 8 / 4 heads of dim 256 in a window of 1024 206 -> 144 us.
 // Error against float64 (2-norm) at those sizes: 4.0e-7 -> 2.9e-7, 3.3e-7 ->
 // 2.5e-7, 5.0e-7 -> 3.5e-7.
 
@@ -487,6 +487,10 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
 #pragma unroll
         for (int x = 0; x < 16; ++x) s[x] = sl[x] = 0.0f;
         h8 kph[2], kpl[2];
+        // (the matrix steps go before the other wave's vector instructions:
+        // 2048 causal tokens at head dim 64 90.5 -> 85.8 us, 512 at 128 42.6
+        // -> 41.8 on MI355X; at 2048 and 128 within 1%)
+        __builtin_amdgcn_s_setprio(1);
         kph[0] = *reinterpret_cast<const h8*>(kl);
         kpl[0] = *reinterpret_cast<const h8*>(kl + C::KPART);
 #pragma unroll
@@ -513,6 +517,7 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        __builtin_amdgcn_s_setprio(0);
 #pragma unroll
         for (int x = 0; x < 16; ++x) s[x] += sl[x];
         // elements 4j .. 4j+3: keys 8j + 4h + r
@@ -597,6 +602,7 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
         };
         v16f o[2];
         h8 vph[2], vpl[2];
+        __builtin_amdgcn_s_setprio(1);
         vph[0] = *reinterpret_cast<const h8*>(value(0));
         vpl[0] = *reinterpret_cast<const h8*>(value(0) + C::VPART);
 #pragma unroll
@@ -631,6 +637,7 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
             }
             __builtin_amdgcn_sched_barrier(0);
         }
+        __builtin_amdgcn_s_setprio(0);
 #pragma unroll
         for (int x = 0; x < 16; ++x)
             acc[NT - 1][x] = __builtin_fmaf(acc[NT - 1][x], alpha, o[(NT - 1) & 1][x]);
