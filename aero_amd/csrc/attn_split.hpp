@@ -717,7 +717,8 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
     }
     if (qok) {
         const float inv = 1.0f / fmaxf(ls, 1e-30f);
-        float* o = p.out + qrow * D + 4 * h;
+        // (64 bits: n_q * n_head rows, up to 2^31 - 1, of D elements)
+        float* o = p.out + (int64_t)qrow * D + 4 * h;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll

@@ -488,3 +488,32 @@ def test_split_rule_matches_general(hip):
         finally:
             tune_set("attn_split", None)
         assert rel_to_scale(got, want) <= RTOL
+
+
+def test_split_output_past_2_32_elements(hip, oracle):
+    """An output of more than 2^32 elements (the first rows, the last ones and
+    those around the 2^32nd element), over 8 keys: nothing wraps onto the
+    first rows."""
+    H, D, S = 33, 128, 8
+    T = 2 ** 32 // (H * D) + 500
+    rng = np.random.default_rng(5)
+    k = rng.standard_normal((S, H, D)).astype(np.float32)
+    v = rng.standard_normal((S, H, D)).astype(np.float32)
+    edge = 2 ** 32 // (H * D)
+    spots = [0, 40, edge - 6, edge + 1, T - 5]
+    q, out = DA.empty((T, H, D)), DA.empty((T, H, D))    # 17 GB each
+    row = H * D * 4
+    ops.fill_f32(q, 0.0)
+    ops.fill_f32(out, -7.0)
+    part = {}
+    for t in spots:
+        part[t] = rng.standard_normal((5, H, D)).astype(np.float32)
+        q.view((5, H, D), offset_bytes=t * row).copy_from(part[t])
+    print(f"split attention T={T} H={H} D={D} S={S}", flush=True)
+    ops.attention(q, DA.from_numpy(k), DA.from_numpy(v), out, T, H, H, D, D, S, 0.125)
+    for t in spots:
+        got = out.view((5, H, D), offset_bytes=t * row).numpy()
+        want = oracle.attention_tiled(part[t], k, v, 0.125, qpos=np.arange(t, t + 5, dtype=np.int32))
+        assert rel_to_scale(got, want) <= RTOL, t
+    q.free()
+    out.free()
