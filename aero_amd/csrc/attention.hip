@@ -418,6 +418,63 @@ __device__ __forceinline__ void merge_tile(const AttnParams& p, float m, float l
     }
 }
 
+// One 16-key tile (first key kb, keys at or past c1 masked) against a wave's
+// 16 queries: scores, running max and sum, value sum.
+template <int DT, int D, int DV>
+__device__ __forceinline__ void mfma_step(const AttnParams& p, const KvTile<DT, D, DV>& tl,
+                                          const float (&qs)[D / 4], int64_t kb, int64_t c1,
+                                          int64_t qp, bool qok, int g, float& m, float& ls,
+                                          v4f (&acc)[DV / 16]) {
+    constexpr int KS = D / 4, VS = DV / 16;
+    v4f s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < KS; j += 2) {
+        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(slice_elem<DT>(tl.k, j), qs[j], s0, 0,
+                                                  0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(slice_elem<DT>(tl.k, j + 1), qs[j + 1],
+                                                  s1, 0, 0, 0);
+    }
+    float sc[4];
+    float tm = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int64_t kj = kb + 4 * g + r;
+        const int64_t kp = p.kpos ? (int64_t)__shfl(tl.kp, 4 * g + r) : kj;
+        const bool keep = qok && kj < c1 && key_kept(kp, qp, p.window);
+        float y = (s0[r] + s1[r]);
+        if constexpr (DT != 0) y *= __shfl(tl.ks, 4 * g + r);
+        sc[r] = keep ? y * p.scale : -INFINITY;
+        tm = fmaxf(tm, sc[r]);
+    }
+    tm = fmaxf(tm, __shfl_xor(tm, 16));
+    tm = fmaxf(tm, __shfl_xor(tm, 32));
+    const float mn = fmaxf(m, tm);
+    const float alpha = (m == -INFINITY) ? 0.0f : expf(m - mn);
+    float pr[4];
+    float psum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        pr[r] = (sc[r] == -INFINITY) ? 0.0f : expf(sc[r] - mn);
+        psum += pr[r];
+        if constexpr (DT != 0) pr[r] *= __shfl(tl.vs, 4 * g + r);
+    }
+    ls = ls * alpha + psum;
+    m = mn;
+    // rescale the rows of query 4g + r by that query's alpha (lane 4g + r)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float ar = __shfl(alpha, 4 * g + r);
+#pragma unroll
+        for (int t = 0; t < VS; ++t) acc[t][r] *= ar;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int t = 0; t < VS; ++t)
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                pr[r], slice_elem<DT>(tl.v[r], t), acc[t], 0, 0, 0);
+}
+
 template <int DT, int D, int DV, bool MERGE_OUT>
 __global__ __launch_bounds__(256) void attn_mfma_kernel(AttnParams p) {
     using Tile = KvTile<DT, D, DV>;
@@ -496,53 +553,7 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(AttnParams p) {
         // (clamped to the chunk's last tile: in bounds, and no branch for the
         // wait counters to merge)
         if constexpr (PF) nx.load(p, c0 + 16 * min(i + istep, tiles_c - 1), c1, g, c, kh);
-        v4f s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < KS; j += 2) {
-            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(slice_elem<DT>(tl.k, j), qs[j], s0, 0,
-                                                      0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(slice_elem<DT>(tl.k, j + 1), qs[j + 1],
-                                                      s1, 0, 0, 0);
-        }
-        float sc[4];
-        float tm = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int64_t kj = kb + 4 * g + r;
-            const int64_t kp = p.kpos ? (int64_t)__shfl(tl.kp, 4 * g + r) : kj;
-            const bool keep = qok && kj < c1 && key_kept(kp, qp, p.window);
-            float y = (s0[r] + s1[r]);
-            if constexpr (DT != 0) y *= __shfl(tl.ks, 4 * g + r);
-            sc[r] = keep ? y * p.scale : -INFINITY;
-            tm = fmaxf(tm, sc[r]);
-        }
-        tm = fmaxf(tm, __shfl_xor(tm, 16));
-        tm = fmaxf(tm, __shfl_xor(tm, 32));
-        const float mn = fmaxf(m, tm);
-        const float alpha = (m == -INFINITY) ? 0.0f : expf(m - mn);
-        float pr[4];
-        float psum = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            pr[r] = (sc[r] == -INFINITY) ? 0.0f : expf(sc[r] - mn);
-            psum += pr[r];
-            if constexpr (DT != 0) pr[r] *= __shfl(tl.vs, 4 * g + r);
-        }
-        ls = ls * alpha + psum;
-        m = mn;
-        // rescale the rows of query 4g + r by that query's alpha (lane 4g + r)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float ar = __shfl(alpha, 4 * g + r);
-#pragma unroll
-            for (int t = 0; t < VS; ++t) acc[t][r] *= ar;
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int t = 0; t < VS; ++t)
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                    pr[r], slice_elem<DT>(tl.v[r], t), acc[t], 0, 0, 0);
+        mfma_step<DT, D, DV>(p, tl, qs, kb, c1, qp, qok, g, m, ls, acc);
         i += istep;
         if (i >= i_hi) break;
         if constexpr (PF)

@@ -10,7 +10,7 @@
 //  * O^T += V^T P^T: A = 32 value dimensions x 16 keys, B = the
 //    probabilities as the scores' accumulator holds them (k-slots 8h + 4b + r
 //    of step s are key 16s + 8b + 4h + r, and V^T is stored in that order).
-// Four waves share the keys of a tile and own 32 query vectors each.
+// The waves share the keys of a tile; a group of queries is 32 vectors.
 //
 // Arithmetic: q (a power of two per query), K and V (a power of two per
 // wave's share of a tile, KW keys) are scaled to below 2^14 and split into
@@ -22,12 +22,17 @@
 // that of the sums; the sums take each step's product with one fma, which
 // carries the change of m and E. Keys that no query of the workgroup
 // keeps become zeros, so what lies in them does not touch the scales.
-// What the split cannot carry is done again in plain fp32 by the wave that
-// owns the rows (attn_rows_plain, about 30 times slower): an infinity (a split
-// makes a NaN of it), sums that are not finite (a NaN among the values reaches
-// queries that do not keep its key), value blocks whose exponents differ by
-// more than 15 or keys and queries whose products pass 2^14 (a small one next
-// to them would keep less than fp32's 24 bits).
+// What the split cannot carry ends the walk, and the workgroup does its 128
+// rows again on fp32 matrix steps (attn_tile_fp32, the sums of
+// attn_mfma_kernel): an infinity (a split makes a NaN of it), sums that are
+// not finite (a NaN among the values reaches queries that do not keep its
+// key), value blocks whose exponents differ by more than 15, or keys and
+// queries whose products pass 2^14 (a small one next to them would keep less
+// than fp32's 24 bits). Time of calls whose every workgroup does so, fp32-step
+// kernel / this one (a row at a time, as it was): 2048 causal tokens, 32 / 8
+// heads of dim 128 467 / 517 us (12.2 ms), of dim 64 256 / 336 us, 8 / 4
+// heads of dim 256 in a window of 1024, whose 128 workgroups leave half of
+// the CUs idle, 235 / 602 us (10.1 ms).
 //
 // Shape. A workgroup owns 128 query vectors of one kv head (32 a wave). At
 // head dims 64 and 128 eight waves walk 128 / 64 keys a step, two waves a
@@ -131,9 +136,9 @@ __device__ __forceinline__ int block_exp(float amax) {
 }
 
 // One wave's n query vectors u0.. of kv head kh over keys [j0, j1), one after
-// the other in plain fp32: the fallback for operands that hold infinities.
-// 64 keys a step, a lane a key for the scores, a lane D / 64 dimensions for
-// the value sum.
+// the other in plain fp32, so that a value that is not finite reaches only the
+// queries that keep its key. 64 keys a step, a lane a key for the scores, a
+// lane D / 64 dimensions for the value sum.
 template <int D>
 __device__ __forceinline__ void attn_rows_plain(const AttnParams& p, int64_t u0, int n, int kh,
                                                 int j0, int j1) {
@@ -176,6 +181,125 @@ __device__ __forceinline__ void attn_rows_plain(const AttnParams& p, int64_t u0,
     }
 }
 
+// Four waves' 16-query tile (query vectors 16 tile .. of kv head kh) over all
+// its keys on the fp32 matrix cores, as attn_mfma_kernel computes it: wave w
+// takes every fourth 16-key tile, the sums meet in LDS (sums; calls are
+// bracketed by barriers, so every wave of the workgroup makes as many). Where
+// a key tile holds keys that some of the queries do not keep, a value that is
+// not finite would reach those too (0 times it): such a query tile is done in
+// plain fp32.
+template <int D>
+struct TileSums {
+    float m[4][16], l[4][16];
+    int leak[4];
+    float acc[4][16][D + 4];
+};
+
+template <int D>
+__device__ __forceinline__ void attn_tile_fp32(const AttnParams& p, int64_t tile, int kh,
+                                               TileSums<D>& sums) {
+    using Tile = KvTile<0, D, D>;
+    constexpr int KS = Tile::KS, VS = Tile::VS;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // (apart from the walk's lane: no register held for it)
+    tid &= 255;
+    const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, c = lane & 15;
+    const int64_t n_vec = p.n_q * p.rep, u0 = tile * 16;
+    const int64_t u = u0 + c;
+    const bool qok = u < n_vec;
+    const int64_t uc = qok ? u : n_vec - 1;
+    const int64_t tq = uc / p.rep;
+    const int64_t qrow = tq * p.n_head + (int64_t)kh * p.rep + uc % p.rep;
+    const int64_t qp = p.qpos ? (int64_t)p.qpos[tq] : tq;
+    float qs[KS];
+#pragma unroll
+    for (int e = 0; e < KS; e += 4) {
+        const v4f f = *reinterpret_cast<const v4f*>(p.q + qrow * D + Tile::kdim(g, e));
+#pragma unroll
+        for (int x = 0; x < 4; ++x) qs[e + x] = qok ? f[x] : 0.0f;
+    }
+    int64_t i_lo = 0, i_hi = u0 < n_vec ? (p.n_kv + 15) / 16 : 0;
+    if (p.kpos == nullptr) {
+        int64_t qmin = qp, qmax = qp;
+#pragma unroll
+        for (int off = 8; off >= 1; off >>= 1) {
+            qmin = min(qmin, (int64_t)__shfl_xor(qmin, off, 16));
+            qmax = max(qmax, (int64_t)__shfl_xor(qmax, off, 16));
+        }
+        i_hi = min(i_hi, max<int64_t>(0, (qmax + 16) / 16));
+        if (p.window > 0) i_lo = max<int64_t>(0, (qmin - p.window + 1) / 16);
+    }
+    float m = -INFINITY, ls = 0.0f;
+    v4f acc[VS];
+#pragma unroll
+    for (int t = 0; t < VS; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+    bool leak = false;
+    for (int64_t i = i_lo + w; i < i_hi; i += 4) {
+        Tile tl;
+        tl.load(p, 16 * i, p.n_kv, g, c, kh);
+        bool part = false;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t kj = 16 * i + 4 * g + r;
+            const int64_t kp = p.kpos ? (int64_t)__shfl(tl.kp, 4 * g + r) : kj;
+            part = part || (qok && !(kj < p.n_kv && key_kept(kp, qp, p.window)));
+        }
+        if (__any(part)) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int t = 0; t < VS; ++t)
+                    leak = leak || !(fabsf(slice_elem<0>(tl.v[r], t)) <= 3.4028235e38f);
+        }
+        mfma_step<0, D, D>(p, tl, qs, 16 * i, p.n_kv, qp, qok, g, m, ls, acc);
+    }
+    ls += __shfl_xor(ls, 16);
+    ls += __shfl_xor(ls, 32);
+    if (g == 0) {
+        sums.m[w][c] = m;
+        sums.l[w][c] = ls;
+    }
+    leak = __any(leak);
+    if (lane == 0) sums.leak[w] = leak;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int t = 0; t < VS; t += 4)
+            *reinterpret_cast<v4f*>(&sums.acc[w][4 * g + r][Tile::vdim(c, t)]) =
+                v4f{acc[t][r], acc[t + 1][r], acc[t + 2][r], acc[t + 3][r]};
+    __syncthreads();
+    if (sums.leak[0] | sums.leak[1] | sums.leak[2] | sums.leak[3]) {
+        attn_rows_plain<D>(p, u0 + 4 * w, (int)max<int64_t>(0, min<int64_t>(4, n_vec - u0 - 4 * w)),
+                           kh, (int)(16 * i_lo), (int)min<int64_t>(16 * i_hi, p.n_kv));
+        return;
+    }
+    // thread (query tid / 16, 4 value elements at a time)
+    const int qi = tid >> 4;
+    if (u0 + qi >= n_vec) return;
+    const int64_t row = (u0 + qi) / p.rep * p.n_head + (int64_t)kh * p.rep + (u0 + qi) % p.rep;
+    float mt = -INFINITY, lt = 0.0f, sc[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) mt = fmaxf(mt, sums.m[x][qi]);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+        sc[x] = sums.m[x][qi] == -INFINITY ? 0.0f : expf(sums.m[x][qi] - mt);
+        lt += sums.l[x][qi] * sc[x];
+    }
+    lt = fmaxf(lt, 1e-30f);
+#pragma unroll 1
+    for (int d = 4 * (tid & 15); d < D; d += 64) {
+        v4f o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const v4f a = *reinterpret_cast<const v4f*>(&sums.acc[x][qi][d]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(a[e], sc[x], o[e]);
+        }
+        *reinterpret_cast<v4f*>(p.out + row * D + d) = v4f{o[0] / lt, o[1] / lt, o[2] / lt, o[3] / lt};
+    }
+}
+
 constexpr float kLog2eLo = 1.92596299e-8f;   // log2(e) - kLog2e
 constexpr int kNoMax = -(1 << 28);     // no key kept yet
 constexpr int kSplitVecs = 128;   // query vectors a workgroup
@@ -188,7 +312,8 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
     __shared__ __attribute__((aligned(16))) _Float16 smem[2][C::BUF];
     __shared__ float s_kf[2][C::NW];   // 2^(e - 14) of each wave's keys
     __shared__ int s_ev[2][C::NW];     // exponent of each wave's values
-    __shared__ int s_bad;              // operands that the split would not carry
+    __shared__ int s_bad[2];           // operands that the split would not carry (by buffer)
+    __shared__ int s_redo;             // sums that are not finite, or not precise
     __shared__ int s_eq;               // the largest query exponent
     __shared__ int s_er[2][C::NW];     // each wave's value exponents: smallest, largest
     __shared__ int32_t s_kp[2][C::KT];
@@ -235,7 +360,7 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
         s_q[0][qg] = qmin;
         s_q[1][qg] = qmax;
         if (qg == 0) {
-            s_bad = 0;
+            s_bad[0] = s_bad[1] = s_redo = 0;
             s_eq = -1000;
         }
     }
@@ -356,14 +481,14 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
             for (int e = 0; e < 8; ++e) av = max3_abs(av, vr[x][e].x, vr[x][e].y);
         wave_max2(ak, av);
         const int ek = block_exp(ak), ev = block_exp(av);
-        if (lane == 0) {
-            s_kf[b][wave] = pow2i(ek - 14);
-            s_ev[b][wave] = ev;
-            if (ev > 128 || ek > ek_lim) s_bad = 1;
-        }
         if (ev > -112) {
             ev_lo = min(ev_lo, ev);
             ev_hi = max(ev_hi, ev);
+        }
+        if (lane == 0) {
+            s_kf[b][wave] = pow2i(ek - 14);
+            s_ev[b][wave] = ev;
+            if (ev > 128 || ek > ek_lim || ev_hi - ev_lo > 15) s_bad[b] = 1;
         }
         fk = pow2i(14 - ek);
         fv = pow2i(14 - ev);
@@ -436,7 +561,7 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
             const float f0 = pow2i(14 - eq);
             if (lq == 0) {
                 s_qe[qg * 32 + r0 + PQ * x] = pow2i(eq - 14);
-                if (eq > 128) s_bad = 1;
+                if (eq > 128) s_bad[0] = 1;
                 atomicMax(&s_eq, eq);
             }
             h2 hi[2], lo[2];
@@ -650,81 +775,97 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
         load(i_lo + 1);
     }
     __syncthreads();
+    // (s_bad[b] is written before the barrier that ends the step of buffer
+    // b ^ 1 and not again before the next one: every wave reads the same)
+    bool redo = false;
     for (int i = i_lo; i < i_hi; ++i) {
         const int b = (i - i_lo) & 1;
+        const int flag = s_bad[b];
         // (past the last tile: zeros, into a buffer that nothing reads)
         scales(b ^ 1, i + 1);
+        redo = __builtin_amdgcn_readfirstlane(flag) != 0;
+        if (redo) break;
         compute(std::true_type{}, b, gk, i);
 #pragma unroll
         for (int sub = gk + C::GK; sub < C::SUBS; sub += C::GK)
             compute(std::false_type{}, b, sub, i);
         __syncthreads();
     }
-
-    if (lane == 0) {
-        s_er[0][wave] = ev_lo;
-        s_er[1][wave] = ev_hi;
-    }
-    if constexpr (C::GK == 1) __syncthreads();
-    // back to natural units, the halves of a column added
-    ls += __shfl_xor(ls, 32);
-    const int back = e_acc - 28;
+    if (!redo) {
+        if (lane == 0) {
+            s_er[0][wave] = ev_lo;
+            s_er[1][wave] = ev_hi;
+        }
+        if constexpr (C::GK == 1) __syncthreads();
+        // back to natural units, the halves of a column added
+        ls += __shfl_xor(ls, 32);
+        const int back = e_acc - 28;
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int x = 0; x < 16; ++x) acc[t][x] = ldexpf(acc[t][x], back);
-    if constexpr (C::GK == 2) {
-        // the second set of waves hands its sums to the first through LDS
-        float* xs = reinterpret_cast<float*>(&smem[0][0]) + qg * (64 * (16 * NT + 2)) + lane;
-        static_assert(4 * 64 * (16 * NT + 2) * 4 <= (int)sizeof(smem), "merge buffer");
-        if (gk == 1) {
-            xs[0] = (float)m;
-            xs[64] = ls;
+            for (int x = 0; x < 16; ++x) acc[t][x] = ldexpf(acc[t][x], back);
+        if constexpr (C::GK == 2) {
+            // the second set of waves hands its sums to the first through LDS
+            float* xs = reinterpret_cast<float*>(&smem[0][0]) + qg * (64 * (16 * NT + 2)) + lane;
+            static_assert(4 * 64 * (16 * NT + 2) * 4 <= (int)sizeof(smem), "merge buffer");
+            if (gk == 1) {
+                xs[0] = (float)m;
+                xs[64] = ls;
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int x = 0; x < 16; ++x) xs[64 * (2 + 16 * t + x)] = acc[t][x];
+            }
+            __syncthreads();
+            if (gk == 0) {
+                const float m0 = (float)m, m1 = xs[0], l1 = xs[64];
+                const float mt = fmaxf(m0, m1);
+                const float w0 = __builtin_amdgcn_exp2f(m0 - mt);
+                const float w1 = __builtin_amdgcn_exp2f(m1 - mt);
+                ls = ls * w0 + l1 * w1;
+                m = max(m, (int)m1);
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int x = 0; x < 16; ++x)
+                        acc[t][x] = acc[t][x] * w0 + xs[64 * (2 + 16 * t + x)] * w1;
+            }
+        }
+#pragma unroll
+        for (int x = 0; x < C::NW; ++x) {
+            ev_lo = min(ev_lo, s_er[0][x]);
+            ev_hi = max(ev_hi, s_er[1][x]);
+        }
+        // (scores past the clamp of m can leave no sum)
+        bool bad = ev_hi - ev_lo > 15 || !(ls <= 3.4028235e38f) || (ls == 0.0f && m != kNoMax);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int x = 0; x < 16; ++x) bad = bad || !(fabsf(acc[t][x]) <= 3.4028235e38f);
+        bad = __any(bad) && gk == 0;
+        if (bad && lane == 0) s_redo = 1;
+        __syncthreads();
+        redo = __builtin_amdgcn_readfirstlane(s_redo) != 0;
+        if (!redo && gk == 0 && qok) {
+            const float inv = 1.0f / fmaxf(ls, 1e-30f);
+            // (64 bits: n_q * n_head rows, up to 2^31 - 1, of D elements)
+            float* o = p.out + (int64_t)qrow * D + 4 * h;
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
-                for (int x = 0; x < 16; ++x) xs[64 * (2 + 16 * t + x)] = acc[t][x];
+                for (int j = 0; j < 4; ++j)
+                    *reinterpret_cast<v4f*>(o + 32 * t + 8 * j) =
+                        v4f{acc[t][4 * j] * inv, acc[t][4 * j + 1] * inv, acc[t][4 * j + 2] * inv,
+                            acc[t][4 * j + 3] * inv};
         }
-        __syncthreads();
-        if (gk == 1) return;
-        const float m0 = (float)m, m1 = xs[0], l1 = xs[64];
-        const float mt = fmaxf(m0, m1);
-        const float w0 = __builtin_amdgcn_exp2f(m0 - mt), w1 = __builtin_amdgcn_exp2f(m1 - mt);
-        ls = ls * w0 + l1 * w1;
-        m = max(m, (int)m1);
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int x = 0; x < 16; ++x)
-                acc[t][x] = acc[t][x] * w0 + xs[64 * (2 + 16 * t + x)] * w1;
     }
-#pragma unroll
-    for (int x = 0; x < C::NW; ++x) {
-        ev_lo = min(ev_lo, s_er[0][x]);
-        ev_hi = max(ev_hi, s_er[1][x]);
-    }
-    // (scores past the clamp of m can leave no sum)
-    bool bad = ev_hi - ev_lo > 15 || s_bad != 0 || !(ls <= 3.4028235e38f) || (ls == 0.0f && m != kNoMax);
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int x = 0; x < 16; ++x) bad = bad || !(fabsf(acc[t][x]) <= 3.4028235e38f);
-    if (__any(bad)) {
-        const int64_t u0 = tile * kSplitVecs + qg * 32;
-        attn_rows_plain<D>(p, u0, (int)max<int64_t>(0, min<int64_t>(32, n_vec - u0)), kh,
-                           KPOS ? 0 : i_lo * C::KT, KPOS ? n_kv : min(n_kv, i_hi * C::KT));
-        return;
-    }
-    if (qok) {
-        const float inv = 1.0f / fmaxf(ls, 1e-30f);
-        // (64 bits: n_q * n_head rows, up to 2^31 - 1, of D elements)
-        float* o = p.out + (int64_t)qrow * D + 4 * h;
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                *reinterpret_cast<v4f*>(o + 32 * t + 8 * j) =
-                    v4f{acc[t][4 * j] * inv, acc[t][4 * j + 1] * inv, acc[t][4 * j + 2] * inv,
-                        acc[t][4 * j + 3] * inv};
+    if (redo) {
+        TileSums<D>* sums = reinterpret_cast<TileSums<D>*>(&smem[0][0]);
+        static_assert(C::GK * sizeof(TileSums<D>) <= sizeof(smem), "sums of the fp32 tiles");
+#pragma unroll 1
+        for (int x = gk; x < kSplitVecs / 16; x += C::GK) {
+            __syncthreads();
+            attn_tile_fp32<D>(p, (int64_t)tile * (kSplitVecs / 16) + x, kh, sums[gk]);
+        }
     }
 }

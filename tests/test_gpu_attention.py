@@ -15,7 +15,7 @@ import pytest
 from conftest import RTOL, bits_equal, golden, rel_to_scale
 from aero_amd import ops
 from aero_amd import transformer_native as TN
-from aero_amd.device import DeviceArray as DA, tune_set
+from aero_amd.device import DeviceArray as DA, Event, tune_set
 
 pytestmark = pytest.mark.gpu
 
@@ -468,6 +468,53 @@ def test_split_non_finite(split_always, oracle, D, bad, where):
         if np.isfinite(general[t, h]).all():
             assert rel_to_scale(got[t, h].astype(np.float64),
                                 general[t, h].astype(np.float64)) <= RTOL
+
+
+@pytest.mark.parametrize("T,H,HK,D,S,window,kpos", [
+    (512, 16, 4, 64, 512, 0, False),
+    (500, 8, 2, 128, 700, 300, False),    # a partial last tile, a window
+    (300, 8, 2, 128, 300, 0, True),
+    (509, 8, 4, 256, 509, 0, False),
+])
+def test_split_redo(split_always, T, H, HK, D, S, window, kpos):
+    """Queries and keys whose products pass what the fp16 parts carry: the
+    workgroups do such rows again on fp32 matrix steps, with the sums of the
+    fp32-step kernel over one chunk (the same partial sums, merged in the same
+    order but for the sum of the probabilities, an fp32 rounding: 1e-7), in a
+    small multiple of its time (on MI355X 1.1 to 3 times, by how much of the
+    chip the workgroups fill; 26 to 65 times with a row at a time)."""
+    rng = np.random.default_rng(T + D)
+    q, k, v = rand_qkv(rng, T, H, HK, D, D, S)
+    for x, up, down in ((q, 3, 7), (k, 7, 3)):
+        x[..., up] *= 256.0
+        x[..., down] /= 256.0
+    dq, dk, dv = DA.from_numpy(q), DA.from_numpy(k), DA.from_numpy(v)
+    qpos = DA.from_numpy(np.arange(S - T, S, dtype=np.int32))
+    kp = DA.from_numpy(rng.permutation(S).astype(np.int32)) if kpos else None
+    print(f"split attention redo T={T} H={H} HK={HK} D={D} S={S}", flush=True)
+    res, ms = [], []
+    for use in (0, 2):
+        tune_set("attn_split", use)
+        tune_set("attn_wgs", 1 if use == 0 else None)    # one chunk
+        out = DA.empty((T, H, D))
+
+        def call():
+            ops.attention(dq, dk, dv, out, T, H, HK, D, D, S, 1.0 / np.sqrt(D), qpos=qpos,
+                          kpos=kp, window=window)
+        call()
+        best = []
+        for _ in range(5):
+            a, b = Event(), Event()
+            a.record()
+            call()
+            b.record()
+            b.synchronize()
+            best.append(a.elapsed_ms(b))
+        res.append(out.numpy().astype(np.float64))
+        ms.append(min(best))
+    assert np.isfinite(res[1]).all()
+    assert np.linalg.norm(res[1] - res[0]) <= 1e-7 * np.linalg.norm(res[0])
+    assert ms[1] <= 10 * ms[0], ms
 
 
 def test_split_rule_matches_general(hip):
