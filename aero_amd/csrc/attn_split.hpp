@@ -26,9 +26,10 @@
 // rows again on fp32 matrix steps (attn_tile_fp32, the sums of
 // attn_mfma_kernel): an infinity (a split makes a NaN of it), sums that are
 // not finite (a NaN among the values reaches queries that do not keep its
-// key), value blocks whose exponents differ by more than 15, or keys and
-// queries whose products pass 2^14 (a small one next to them would keep less
-// than fp32's 24 bits). Time of calls whose every workgroup does so, fp32-step
+// key), rows of V whose exponents differ by more than kSpread, in a block or
+// between blocks (a query may keep the small ones alone), or keys and queries
+// whose products pass 2^14 (a small one next to them would keep less than
+// fp32's 24 bits). Time of calls whose every workgroup does so, fp32-step
 // kernel / this one (a row at a time, as it was): 2048 causal tokens, 32 / 8
 // heads of dim 128 467 / 517 us (12.2 ms), of dim 64 256 / 336 us, 8 / 4
 // heads of dim 256 in a window of 1024, whose 128 workgroups leave half of
@@ -96,6 +97,10 @@ __device__ __forceinline__ float max3_abs(float a, float b, float c) {
     asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(a) : "v"(b), "v"(c));
     return a;
 }
+__device__ __forceinline__ float min3_abs(float a, float b, float c) {
+    asm("v_min3_f32 %0, |%0|, |%1|, |%2|" : "+v"(a) : "v"(b), "v"(c));
+    return a;
+}
 
 // the largest a and b over each 16-lane row, in every lane of it (a DPP
 // operand may be read two instructions after it is written)
@@ -115,6 +120,18 @@ __device__ __forceinline__ void row_max2(float& a, float& b) {
         "s_nop 1"
         : "+v"(a), "+v"(b));
 }
+__device__ __forceinline__ float lane_value(float x, int lane) {
+    return __builtin_bit_cast(float,
+                              __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
+// the same for each half of the wave, in its lane 31 (row 1 has met row 0)
+__device__ __forceinline__ void half_max2(float& a, float& b) {
+    row_max2(a, b);
+    asm("v_max_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n"
+        "v_max_f32_dpp %1, %1, %1 row_bcast:15 row_mask:0xa bank_mask:0xf\n"
+        "s_nop 1"
+        : "+v"(a), "+v"(b));
+}
 // the largest a and b over the wave, wave-uniform
 __device__ __forceinline__ void wave_max2(float& a, float& b) {
     row_max2(a, b);
@@ -125,8 +142,8 @@ __device__ __forceinline__ void wave_max2(float& a, float& b) {
         "v_max_f32_dpp %1, %1, %1 row_bcast:31 row_mask:0xc bank_mask:0xf\n"
         "s_nop 1"
         : "+v"(a), "+v"(b));
-    a = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, a), 63));
-    b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, b), 63));
+    a = lane_value(a, 63);
+    b = lane_value(b, 63);
 }
 
 // e with |x| < 2^e for a block's largest |x|, clamped so that 2^(14 - e) and
@@ -303,6 +320,11 @@ __device__ __forceinline__ void attn_tile_fp32(const AttnParams& p, int64_t tile
 constexpr float kLog2eLo = 1.92596299e-8f;   // log2(e) - kLog2e
 constexpr int kNoMax = -(1 << 28);     // no key kept yet
 constexpr int kSplitVecs = 128;   // query vectors a workgroup
+// Largest difference of the exponents of two rows of V that a workgroup may
+// keep. A query may keep small rows alone, or large ones with probabilities
+// that make them as small: what the parts drop, 2^-39 of the largest, is then
+// 2^-21 of the query's result, which is what the fp32 steps' sums leave.
+constexpr int kSpread = 18;
 
 template <int D, bool KPOS>
 __global__ __launch_bounds__(64 * SplitCfg<D>::NW)
@@ -482,13 +504,50 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
         wave_max2(ak, av);
         const int ek = block_exp(ak), ev = block_exp(av);
         if (ev > -112) {
-            ev_lo = min(ev_lo, ev);
+            // The smallest of the rows (keys) of V that are not zeros. In most
+            // blocks one lane (of each half at head dim 64) sees in its first
+            // dimension that all are within 2^-5 of the largest; else (keys
+            // that nothing keeps among them) the rows' own maxima.
+            float mn = vr[0][0].x;
+            mn = min3_abs(mn, vr[0][1].x, vr[0][2].x);
+            mn = min3_abs(mn, vr[0][3].x, vr[0][4].x);
+            mn = min3_abs(mn, vr[0][5].x, vr[0][6].x);
+            mn = min3_abs(mn, vr[0][7].x, vr[0][7].x);
+            const uint64_t near = __ballot(mn >= av * 0.03125f);
+            int lo = ev - 5;
+            if (D == 64 ? (uint32_t)near == 0 || (near >> 32) == 0 : near == 0) {
+                asm volatile("");   // (a branch)
+                float low = av;
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {
+                    float r0 = 0.0f, r1 = 0.0f;
+#pragma unroll
+                    for (int x = 0; x < C::CV; ++x) {
+                        r0 = max3_abs(r0, vr[x][e].x, vr[x][e].y);
+                        r1 = max3_abs(r1, vr[x][e + 1].x, vr[x][e + 1].y);
+                    }
+                    if constexpr (D == 64) {
+                        half_max2(r0, r1);
+                        const float o0 = lane_value(r0, 31), o1 = lane_value(r1, 31);
+                        low = fminf(low, o0 > 0.0f ? o0 : av);
+                        low = fminf(low, o1 > 0.0f ? o1 : av);
+                        r0 = lane_value(r0, 63);
+                        r1 = lane_value(r1, 63);
+                    } else {
+                        wave_max2(r0, r1);
+                    }
+                    low = fminf(low, r0 > 0.0f ? r0 : av);
+                    low = fminf(low, r1 > 0.0f ? r1 : av);
+                }
+                lo = __builtin_amdgcn_readfirstlane(block_exp(low));
+            }
+            ev_lo = min(ev_lo, lo);
             ev_hi = max(ev_hi, ev);
         }
         if (lane == 0) {
             s_kf[b][wave] = pow2i(ek - 14);
             s_ev[b][wave] = ev;
-            if (ev > 128 || ek > ek_lim || ev_hi - ev_lo > 15) s_bad[b] = 1;
+            if (ev > 128 || ek > ek_lim || ev_hi - ev_lo > kSpread) s_bad[b] = 1;
         }
         fk = pow2i(14 - ek);
         fv = pow2i(14 - ev);
@@ -837,7 +896,7 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
             ev_hi = max(ev_hi, s_er[1][x]);
         }
         // (scores past the clamp of m can leave no sum)
-        bool bad = ev_hi - ev_lo > 15 || !(ls <= 3.4028235e38f) || (ls == 0.0f && m != kNoMax);
+        bool bad = ev_hi - ev_lo > kSpread || !(ls <= 3.4028235e38f) || (ls == 0.0f && m != kNoMax);
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll

@@ -470,6 +470,31 @@ def test_split_non_finite(split_always, oracle, D, bad, where):
                                 general[t, h].astype(np.float64)) <= RTOL
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("T,S,window,turned,up", [
+    (8, 8, 0, False, 40),      # a few keys
+    (100, 100, 3, False, 40),  # queries that keep none of the large rows
+    (100, 100, 3, True, 40),   # the same, keys stored last to first
+    (100, 100, 3, False, 24),
+    (100, 100, 3, False, 14),
+])
+def test_split_value_rows(split_always, oracle, D, T, S, window, turned, up):
+    """Every fourth row of V 2^up above the others, so that every block of keys
+    that shares a scale holds both: a query that keeps small rows alone gets
+    them whole (each query against its own scale)."""
+    rng = np.random.default_rng(D + T + up)
+    q, k, v = rand_qkv(rng, T, 4, 2, D, D, S)
+    v[3::4] *= 2.0 ** up
+    qpos = np.arange(S - T, S, dtype=np.int32)
+    kpos = np.arange(S, dtype=np.int32)[::-1] if turned else None
+    scale = 1.0 / np.sqrt(D)
+    print(f"split attention D={D} T={T} S={S} V rows 2^{up} apart", flush=True)
+    got = gpu_attention(q, k, v, scale, qpos=qpos, kpos=kpos, window=window)
+    want = oracle.attention_tiled(q, k, v, scale, qpos=qpos, kpos=kpos, window=window or None)
+    for t in range(T):
+        assert rel_to_scale(got[t], want[t]) <= RTOL, t
+
+
 @pytest.mark.parametrize("T,H,HK,D,S,window,kpos", [
     (512, 16, 4, 64, 512, 0, False),
     (500, 8, 2, 128, 700, 300, False),    # a partial last tile, a window
