@@ -27,7 +27,8 @@
 // attn_mfma_kernel): an infinity (a split makes a NaN of it), sums that are
 // not finite (a NaN among the values reaches queries that do not keep its
 // key), rows of V whose exponents differ by more than kSpread, in a block or
-// between blocks (a query may keep the small ones alone), or keys and queries
+// between blocks (a query may keep the small ones alone), dimensions of V that
+// do by more than kSpreadCh (known at the end of the walk), or keys and queries
 // whose products pass 2^14 (a small one next to them would keep less than
 // fp32's 24 bits). Time of calls whose every workgroup does so, fp32-step
 // kernel / this one (a row at a time, as it was): 2048 causal tokens, 32 / 8
@@ -325,6 +326,11 @@ constexpr int kSplitVecs = 128;   // query vectors a workgroup
 // that make them as small: what the parts drop, 2^-39 of the largest, is then
 // 2^-21 of the query's result, which is what the fp32 steps' sums leave.
 constexpr int kSpread = 18;
+// The same of two dimensions of V, by each one's largest value in the walk:
+// what is dropped meets every key, and is 2^-25 of the dimension's scale at
+// this ratio (error of the worst of 128 dimensions, fp32 steps / split, one of
+// them 2^14 above the others 3.1e-7 / 2.9e-7, 2^16 3.1 / 5.0, 2^20 3.3 / 99).
+constexpr int kSpreadCh = 14;
 
 template <int D, bool KPOS>
 __global__ __launch_bounds__(64 * SplitCfg<D>::NW)
@@ -338,6 +344,7 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
     __shared__ int s_redo;             // sums that are not finite, or not precise
     __shared__ int s_eq;               // the largest query exponent
     __shared__ int s_er[2][C::NW];     // each wave's value exponents: smallest, largest
+    __shared__ uint32_t s_ch[D];       // the largest |value| of each dimension (its bits)
     __shared__ int32_t s_kp[2][C::KT];
     __shared__ int32_t s_q[2][4];
     __shared__ float s_qe[kSplitVecs];   // 2^(e - 14) of each query
@@ -378,6 +385,7 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
     }
     qmin = __builtin_amdgcn_readfirstlane(qmin);
     qmax = __builtin_amdgcn_readfirstlane(qmax);
+    for (int d = threadIdx.x; d < D; d += 64 * C::NW) s_ch[d] = 0;
     if (lane == 0 && gk == 0) {
         s_q[0][qg] = qmin;
         s_q[1][qg] = qmax;
@@ -456,6 +464,9 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
     // zeroed, the scales
     float fk, fv;
     int ek_lim = 0, ev_lo = 1000, ev_hi = -1000;
+    float vch[C::CV][2];   // the largest value of each of the lane's dimensions
+#pragma unroll
+    for (int x = 0; x < C::CV; ++x) vch[x][0] = vch[x][1] = 0.0f;
     auto scales = [&](int b, int i) __attribute__((always_inline)) {
         const int first = i * C::KT + wave * C::KW;
         // keys of the tile that no query of the workgroup keeps become zeros
@@ -497,10 +508,19 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
 #pragma unroll
             for (int y = 0; y < 8; y += 2)
                 ak = max3_abs(ak, kr[x][y >> 2][y & 3], kr[x][y >> 2][(y & 3) + 1]);
+        // (a dimension's largest first: the lane keeps the walk's)
 #pragma unroll
-        for (int x = 0; x < C::CV; ++x)
+        for (int x = 0; x < C::CV; ++x) {
+            float c[2] = {0.0f, 0.0f};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) av = max3_abs(av, vr[x][e].x, vr[x][e].y);
+            for (int e = 0; e < 8; e += 2) {
+                c[0] = max3_abs(c[0], vr[x][e].x, vr[x][e + 1].x);
+                c[1] = max3_abs(c[1], vr[x][e].y, vr[x][e + 1].y);
+            }
+            av = max3(av, c[0], c[1]);
+            vch[x][0] = max3(vch[x][0], c[0], c[0]);
+            vch[x][1] = max3(vch[x][1], c[1], c[1]);
+        }
         wave_max2(ak, av);
         const int ek = block_exp(ak), ev = block_exp(av);
         if (ev > -112) {
@@ -855,6 +875,10 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
             s_er[0][wave] = ev_lo;
             s_er[1][wave] = ev_hi;
         }
+#pragma unroll
+        for (int x = 0; x < 2 * C::CV; ++x)
+            atomicMax(&s_ch[vd + 128 * (x >> 1) + (x & 1)],
+                      __builtin_bit_cast(uint32_t, vch[x >> 1][x & 1]));
         if constexpr (C::GK == 1) __syncthreads();
         // back to natural units, the halves of a column added
         ls += __shfl_xor(ls, 32);
@@ -895,8 +919,15 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
             ev_lo = min(ev_lo, s_er[0][x]);
             ev_hi = max(ev_hi, s_er[1][x]);
         }
+        // (a dimension of V far below the others; one of zeros is exact)
+        bool faint = false;
+#pragma unroll
+        for (int d = lane; d < D; d += 64) {
+            const uint32_t c = s_ch[d];
+            faint = faint || (c != 0 && ev_hi - block_exp(__builtin_bit_cast(float, c)) > kSpreadCh);
+        }
         // (scores past the clamp of m can leave no sum)
-        bool bad = ev_hi - ev_lo > kSpread || !(ls <= 3.4028235e38f) || (ls == 0.0f && m != kNoMax);
+        bool bad = faint || ev_hi - ev_lo > kSpread || !(ls <= 3.4028235e38f) || (ls == 0.0f && m != kNoMax);
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll

@@ -495,6 +495,32 @@ def test_split_value_rows(split_always, oracle, D, T, S, window, turned, up):
         assert rel_to_scale(got[t], want[t]) <= RTOL, t
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("up", [12, 18, 24, 60])
+def test_split_value_channels(split_always, D, up):
+    """A dimension of V 2^up above the others, with dimensions of zeros (a
+    padded head) among these: each is as good against its own scale as without
+    it (2-norm against float64 2.6e-7 to 4e-7 on either kernel; 2^-25 of the
+    dimension's scale more at the ratio that the split takes)."""
+    rng = np.random.default_rng(D + up)
+    T, H, HK, S = 150, 4, 2, 150
+    q, k, v = rand_qkv(rng, T, H, HK, D, D, S)
+    v[:, 1, 5] *= 2.0 ** up
+    v[:, :, D - 7:] = 0.0
+    scale = 1.0 / np.sqrt(D)
+    print(f"split attention D={D} a V channel 2^{up} up", flush=True)
+    got = gpu_attention(q, k, v, scale, qpos=np.arange(T, dtype=np.int32)).astype(np.float64)
+    mask = np.arange(S)[None] > np.arange(T)[:, None]
+    for h in range(H):
+        s = q[:, h].astype(np.float64) @ k[:, h // 2].T.astype(np.float64) * np.float32(scale)
+        s[mask] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        want = p @ v[:, h // 2].astype(np.float64) / p.sum(1, keepdims=True)
+        assert not got[:, h, D - 7:].any()
+        err = np.linalg.norm(got[:, h] - want, axis=0)[:D - 7]
+        assert (err <= 1e-6 * np.linalg.norm(want, axis=0)[:D - 7]).all(), err.max()
+
+
 @pytest.mark.parametrize("T,H,HK,D,S,window,kpos", [
     (512, 16, 4, 64, 512, 0, False),
     (500, 8, 2, 128, 700, 300, False),    # a partial last tile, a window
