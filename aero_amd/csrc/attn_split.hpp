@@ -29,8 +29,7 @@
 // key), rows of V whose exponents differ by more than kSpread, in a block or
 // between blocks (a query may keep the small ones alone), dimensions of V that
 // do by more than kSpreadCh (known at the end of the walk), or keys and queries
-// whose products pass 2^14 (a small one next to them would keep less than
-// fp32's 24 bits). Time of calls whose every workgroup does so, fp32-step
+// whose products pass 2^kScoreExp. Time of calls whose every workgroup does so, fp32-step
 // kernel / this one (a row at a time, as it was): 2048 causal tokens, 32 / 8
 // heads of dim 128 467 / 517 us (12.2 ms), of dim 64 256 / 336 us, 8 / 4
 // heads of dim 256 in a window of 1024, whose 128 workgroups leave half of
@@ -331,6 +330,13 @@ constexpr int kSpread = 18;
 // this ratio (error of the worst of 128 dimensions, fp32 steps / split, one of
 // them 2^14 above the others 3.1e-7 / 2.9e-7, 2^16 3.1 / 5.0, 2^20 3.3 / 99).
 constexpr int kSpreadCh = 14;
+// The largest exponent of a query's largest value times a block's largest key
+// value (log2 units). What the parts of a small q drop meets a large K and the
+// reverse: 2^-39 of that product a dimension, so up to D / 2 * 2^-27 (2^-20 of
+// a probability at dim 256) if large and small meet in every dimension and all
+// roundings have one sign. Such a case at dim 256, error of the result on fp32
+// steps / split: product 2^12 3e-8 / 2.7e-7, 2^14 6e-9 / 1.2e-6.
+constexpr int kScoreExp = 12;
 
 template <int D, bool KPOS>
 __global__ __launch_bounds__(64 * SplitCfg<D>::NW)
@@ -662,7 +668,7 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
             qlo[st] = *reinterpret_cast<const h8*>(qf + 16 * st + QPART);
         }
         qsc = s_qe[qg * 32 + n];
-        ek_lim = __builtin_amdgcn_readfirstlane(min(14 - s_eq, 128));
+        ek_lim = __builtin_amdgcn_readfirstlane(min(kScoreExp - s_eq, 128));
         __syncthreads();
     }
 
@@ -927,7 +933,8 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
             faint = faint || (c != 0 && ev_hi - block_exp(__builtin_bit_cast(float, c)) > kSpreadCh);
         }
         // (scores past the clamp of m can leave no sum)
-        bool bad = faint || ev_hi - ev_lo > kSpread || !(ls <= 3.4028235e38f) || (ls == 0.0f && m != kNoMax);
+        bool bad = faint || ev_hi - ev_lo > kSpread || !(ls <= 3.4028235e38f) ||
+                   (ls == 0.0f && m != kNoMax);
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll

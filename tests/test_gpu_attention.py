@@ -521,6 +521,37 @@ def test_split_value_channels(split_always, D, up):
         assert (err <= 1e-6 * np.linalg.norm(want, axis=0)[:D - 7]).all(), err.max()
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("e", [10, 12, 13, 14])
+def test_split_score_products(split_always, D, e):
+    """Large q values against small K values whose parts drop a remainder of
+    one sign, next to K values (met by zeros of q) that set the scale, the
+    maxima's product just below 2^e log2 units: at most D / 2 * 2^(e - 39) off
+    in the scores, D / 2 * 2^-27 where the split takes them (e <= 12), so that
+    times ln 2 / 2 in a result that is a mean of zeros and ones near 1/2 and
+    twice that relative to it; the kernels' own 1e-7 on top."""
+    rng = np.random.default_rng(0)
+    S, T = 64, 40
+    scale = 1.0 / np.sqrt(D)
+    up = 2.0 ** (e - e // 2)
+    sign = np.where(rng.permutation(S) % 2 == 0, 1.0, -1.0)
+    q = np.zeros((T, 1, D), np.float32)
+    q[..., :D // 2] = 0.99 * 2.0 ** (e // 2) / (scale * np.log2(np.e))
+    k = np.zeros((S, 1, D), np.float32)
+    k[..., D // 2:] = 0.99 * up
+    # (in units of up / 2^14: 2^-5 and up to 2^-18 more, 0.48 of the last fp16 bit over)
+    k[..., :D // 2] = (2.0 ** -5 + rng.integers(-64, 64, (S, 1, D // 2)) * 2.0 ** -24 +
+                       sign[:, None, None] * 0.48 * 2.0 ** -24) * up / 2 ** 14
+    v = np.zeros((S, 1, D), np.float32)
+    v[sign > 0] = 1.0
+    print(f"split attention D={D} products 2^{e}", flush=True)
+    got = gpu_attention(q, k, v, scale, qpos=np.full(T, S, np.int32))[:, 0].astype(np.float64)
+    s = q[:, 0].astype(np.float64) @ k[:, 0].T.astype(np.float64) * np.float32(scale)
+    p = np.exp(s - s.max(1, keepdims=True))
+    want = p @ v[:, 0].astype(np.float64) / p.sum(1, keepdims=True)
+    assert np.abs(got - want).max() <= (D / 2 * 2.0 ** -27 * np.log(2) + 1e-7) * np.abs(want).max()
+
+
 @pytest.mark.parametrize("T,H,HK,D,S,window,kpos", [
     (512, 16, 4, 64, 512, 0, False),
     (500, 8, 2, 128, 700, 300, False),    # a partial last tile, a window
