@@ -400,13 +400,18 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams p) {
 // l%16: d is lane-local. Lane l supplies columns 8(l/16) .. +7 of token l%16
 // and of row l%16, loaded as they lie.)
 //
-// The four waves of a workgroup own the same NT x 16 rows and MT x 16 tokens
-// and take every fourth block; their sums meet in LDS once at the end, so
+// d comes after the sum over the block, and the smallest part of an x below
+// 2^-110 is below bf16's last bit: a step whose x lies outside 2^-100 .. 2^100
+// is computed on x times a power of two a token.
+//
+// The eight waves of a workgroup own the same NT x 16 rows and MT x 16 tokens
+// and take every eighth block; their sums meet in LDS once at the end, so
 // the loop has no barrier and no LDS traffic, and short rows (896 columns: 28
-// blocks) still keep four waves busy. A part of x costs vector instructions
+// blocks) still keep eight waves busy. A part of x costs vector instructions
 // per row tile instead (about as long as the matrix steps at NT = 2).
 // Measured on MI355X against the fp32 matrix steps of gemm_kernel (2.7 times
 // the matrix time, 128-column chunks between barriers): see launch_q8.
+constexpr uint32_t kQ8Large = 227u << 23, kQ8Small = 27u << 23;   // 2^100, 2^-100
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 typedef uint32_t u3w __attribute__((ext_vector_type(3), aligned(4)));
 
@@ -427,10 +432,11 @@ __device__ __forceinline__ bf8v q8_bf16(uint32_t w0, uint32_t w1) {
     return __builtin_bit_cast(bf8v, make_uint4(o[0], o[1], o[2], o[3]));
 }
 
-// 8 floats as three bf16 parts (part 0 the largest); an infinity keeps part 0
+// 8 floats as three bf16 parts (part 0 the largest); with INF an infinity
+// keeps part 0 alone
+template <bool INF>
 __device__ __forceinline__ void bf16_parts(const float (&x)[8], bf8v (&p)[3]) {
     float r[3][8];
-    float big = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const float h = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x[i]) & 0xFFFF0000u);
@@ -439,14 +445,7 @@ __device__ __forceinline__ void bf16_parts(const float (&x)[8], bf8v (&p)[3]) {
         const float m =
             __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r[1][i]) & 0xFFFF0000u);
         r[2][i] = r[1][i] - m;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; i += 2)
-        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(big) : "v"(x[i]), "v"(x[i + 1]));
-    if (__any(big > 3.4028235e38f)) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (fabsf(x[i]) > 3.4028235e38f) r[1][i] = r[2][i] = 0.0f;
+        if (INF && fabsf(x[i]) > 3.4028235e38f) r[1][i] = r[2][i] = 0.0f;
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -457,6 +456,15 @@ __device__ __forceinline__ void bf16_parts(const float (&x)[8], bf8v (&p)[3]) {
                                          __builtin_bit_cast(uint32_t, r[k][2 * i]), 0x07060302u);
         p[k] = __builtin_bit_cast(bf8v, make_uint4(o[0], o[1], o[2], o[3]));
     }
+}
+
+// the largest magnitude of 8 floats (a NaN is ignored: it shows in the sums)
+__device__ __forceinline__ float largest(const float (&x)[8]) {
+    float big = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; i += 2)
+        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(big) : "v"(x[i]), "v"(x[i + 1]));
+    return big;
 }
 
 template <int MT, int NT, int KW>
@@ -479,7 +487,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_q8_kernel(GemmParams p) {
     for (int m = 0; m < MT; ++m)
         xp[m] = p.x + (int64_t)min(t0 + 16 * m + c, p.n_tok - 1) * p.x_stride + 8 * g;
 
-    float4 xa[MT][2];
+    v4f xa[MT][2];
     u3w wq[NT];
     uint32_t wd[NT];
     // the codes lie 2 bytes off a dword in every other block (and row, where
@@ -489,8 +497,8 @@ __global__ __launch_bounds__(64 * KW) void gemm_q8_kernel(GemmParams p) {
         b = min(b, nb - 1);
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            xa[m][0] = *reinterpret_cast<const float4*>(xp[m] + 32 * b);
-            xa[m][1] = *reinterpret_cast<const float4*>(xp[m] + 32 * b + 4);
+            xa[m][0] = *reinterpret_cast<const v4f*>(xp[m] + 32 * b);
+            xa[m][1] = *reinterpret_cast<const v4f*>(xp[m] + 32 * b + 4);
         }
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
@@ -522,26 +530,61 @@ __global__ __launch_bounds__(64 * KW) void gemm_q8_kernel(GemmParams p) {
                             __builtin_amdgcn_alignbyte(wq[j][2], wq[j][1], sh));
             d[j] = half_bits_to_float(wd[j]);
         }
-        bf8v xb[MT][3];
+        float x[MT][8];
+        uint32_t hi = 0, lo = ~0u;    // bits of the largest values; zeros pass
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            const float x[8] = {xa[m][0].x, xa[m][0].y, xa[m][0].z, xa[m][0].w,
-                                xa[m][1].x, xa[m][1].y, xa[m][1].z, xa[m][1].w};
-            bf16_parts(x, xb[m]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[m][i] = xa[m][i >> 2][i & 3];
+            const uint32_t u = __builtin_bit_cast(uint32_t, largest(x[m]));
+            hi = max(hi, u);
+            lo = min(lo, u - 1);
         }
-        load(b + KW);
+        bf8v xb[MT][3];
+        auto product = [&](int m, int j) __attribute__((always_inline)) {
+            v4f part = {0.f, 0.f, 0.f, 0.f};
+            part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xb[m][2], wb[j], part, 0, 0, 0);
+            part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xb[m][1], wb[j], part, 0, 0, 0);
+            return __builtin_amdgcn_mfma_f32_16x16x32_bf16(xb[m][0], wb[j], part, 0, 0, 0);
+        };
+        if (!__any(hi > kQ8Large || lo < kQ8Small)) {
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
+            for (int m = 0; m < MT; ++m) bf16_parts<false>(x[m], xb[m]);
+            load(b + KW);
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                v4f part = {0.f, 0.f, 0.f, 0.f};
-                part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xb[m][2], wb[j], part, 0, 0, 0);
-                part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xb[m][1], wb[j], part, 0, 0, 0);
-                part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xb[m][0], wb[j], part, 0, 0, 0);
+            for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    acc[m][j][v] = __builtin_fmaf(part[v], d[j], acc[m][j][v]);
+                for (int j = 0; j < NT; ++j) {
+                    const v4f part = product(m, j);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        acc[m][j][v] = __builtin_fmaf(part[v], d[j], acc[m][j][v]);
+                }
+        } else {
+            // a token's 32 values times the power of two 2^-e that brings
+            // the largest near 1; half of 2^e goes to the sum, half to d
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                uint32_t t = __builtin_bit_cast(uint32_t, largest(x[m]));
+                t = max(t, (uint32_t)__shfl_xor((int)t, 16));
+                t = max(t, (uint32_t)__shfl_xor((int)t, 32));
+                const int e = (int)(t >> 23) - 126;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[m][i] = ldexpf(x[m][i], -e);
+                bf16_parts<true>(x[m], xb[m]);
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    const v4f part = product(m, j);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int ev = __shfl(e, 4 * g + v);
+                        acc[m][j][v] = __builtin_fmaf(ldexpf(part[v], ev / 2),
+                                                      ldexpf(d[j], ev - ev / 2), acc[m][j][v]);
+                    }
+                }
             }
+            load(b + KW);
+        }
     }
 
 #pragma unroll

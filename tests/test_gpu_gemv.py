@@ -235,6 +235,53 @@ def test_gemm_q8_non_finite(hip, oracle):
         assert np.array_equal(np.sign(got[t]), np.sign(want[t]), equal_nan=True)
 
 
+@pytest.mark.parametrize("tile", range(1, 8))
+@pytest.mark.parametrize("e", [-140, -121, -113, 110, 122, 126])
+def test_gemm_q8_far_x(hip, tile, e):
+    """x near either end of fp32's range against float64: every other token's
+    values are 2^e (ordinary tokens between them, and an ordinary group of 8
+    columns in each), d such that no result leaves that range. x, codes and d are exact; a step's sum of 32 and 28
+    such steps leave 60 roundings of 2^-24 of the sum of magnitudes at most."""
+    rng = np.random.default_rng(tile)
+    n_rows, n_cols, n_tok = 70, 896, 66
+    d = 2.0 ** -20 if e > 0 else 2.0 ** 10
+    code = rng.integers(-127, 128, (n_rows, n_cols // 32, 32), dtype=np.int8)
+    raw = np.empty((n_rows, n_cols // 32, 34), np.uint8)
+    raw[..., :2] = np.full((n_rows, n_cols // 32, 1), d, np.float16).view(np.uint8)
+    raw[..., 2:] = code.view(np.uint8)
+    X = rng.standard_normal((n_tok, n_cols)).clip(-3.9, 3.9).astype(np.float32)
+    far = np.arange(n_tok) % 2 == 1
+    X[far] = np.ldexp(X[far], e - 1 if e == 126 else e)
+    X[far, 40:48] = rng.standard_normal((far.sum(), 8))
+    y = DA.empty((n_tok, n_rows))
+    print(f"gemm_q8 tile={tile} x 2^{e}", flush=True)
+    tune_set("gemm_q8_tile", tile)
+    try:
+        ops.matvec(W.Q8_0, DA.from_numpy(raw.reshape(-1)), DA.from_numpy(X), y, n_rows, n_cols,
+                   n_tok, split=False)
+    finally:
+        tune_set("gemm_q8_tile", None)
+    w = code.astype(np.float64).reshape(n_rows, n_cols) * d
+    want = X.astype(np.float64) @ w.T
+    size = np.abs(X.astype(np.float64)) @ np.abs(w.T)
+    got = y.numpy().astype(np.float64)
+    assert np.isfinite(got).all()
+    assert (np.abs(got - want) <= 60 * 2.0 ** -24 * size).all()
+    if e < 0:        # without the ordinary columns a tiny token stands alone
+        X[far, 40:48] = np.ldexp(X[far, 40:48], e)
+        want = X.astype(np.float64) @ w.T
+        tune_set("gemm_q8_tile", tile)
+        try:
+            ops.matvec(W.Q8_0, DA.from_numpy(raw.reshape(-1)), DA.from_numpy(X), y, n_rows,
+                       n_cols, n_tok, split=False)
+        finally:
+            tune_set("gemm_q8_tile", None)
+        got = y.numpy().astype(np.float64)
+        lim = np.maximum(60 * 2.0 ** -24 * (np.abs(X.astype(np.float64)) @ np.abs(w.T)),
+                         30 * 2.0 ** -149)
+        assert (np.abs(got - want) <= lim).all()
+
+
 @pytest.mark.parametrize("n_rows,n_cols,n_tok", [(896, 4864, 16), (896, 4864, 100),
                                                  (1024, 4096, 12), (1024, 4096, 13),
                                                  (512, 2048, 5), (130, 5120, 5), (130, 2304, 5)])
