@@ -413,7 +413,6 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmParams p) {
 // the matrix time, 128-column chunks between barriers): see launch_q8.
 constexpr uint32_t kQ8Large = 227u << 23, kQ8Small = 27u << 23;   // 2^100, 2^-100
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
-typedef uint32_t u3w __attribute__((ext_vector_type(3), aligned(4)));
 
 // 8 int8 codes (two dwords) as bf16: each byte offset by 128, converted and
 // shifted back (exact), the upper halves of the floats packed
@@ -488,11 +487,11 @@ __global__ __launch_bounds__(64 * KW) void gemm_q8_kernel(GemmParams p) {
         xp[m] = p.x + (int64_t)min(t0 + 16 * m + c, p.n_tok - 1) * p.x_stride + 8 * g;
 
     v4f xa[MT][2];
-    u3w wq[NT];
+    uint32_t wq[NT][3];
     uint32_t wd[NT];
     // the codes lie 2 bytes off a dword in every other block (and row, where
-    // their number is odd): the dwords around them, shifted into place; the
-    // last dword holds at least two of the codes
+    // their number is odd): two dwords from the one that holds the first code,
+    // and the last two codes, which lie in neither there; shifted into place
     auto load = [&](int b) __attribute__((always_inline)) {
         b = min(b, nb - 1);
 #pragma unroll
@@ -504,11 +503,10 @@ __global__ __launch_bounds__(64 * KW) void gemm_q8_kernel(GemmParams p) {
         for (int j = 0; j < NT; ++j) {
             const uint8_t* e = wp[j] + (int64_t)34 * b;
             const uintptr_t a = reinterpret_cast<uintptr_t>(e + 2 + 8 * g);
-            // (aligned: dwords 0 and 1, and dword 1 again; else 0, 1 and 2)
             const uint32_t* d = reinterpret_cast<const uint32_t*>(a & ~uintptr_t(3));
             wq[j][0] = d[0];
             wq[j][1] = d[1];
-            wq[j][2] = d[(a & 2) ? 2 : 1];
+            wq[j][2] = *reinterpret_cast<const uint16_t*>(e + 8 + 8 * g);
             wd[j] = *reinterpret_cast<const uint16_t*>(e);
         }
     };

@@ -156,3 +156,37 @@ def test_rows_not_admitted():
     # Q8_0 8-byte rows without the padding after the last row
     rb = 896 // 32 * 34
     assert not lanes64_ok(W.Q8_0, rb, 3, 3 * rb)
+
+
+def q8_gemm_windows(rowp, n_blk, old=False):
+    """(first byte, one past the last byte) of the loads of gemm_q8_kernel
+    (aero_amd/csrc/gemm.hip) in a row at rowp, for every block and lane group
+    g: two dwords from the one that holds code 8g, two bytes at codes 8g + 6
+    and 7, the scale. The old third piece was the dword after the two where
+    the codes lie off a dword."""
+    e = rowp + 34 * np.arange(n_blk, dtype=np.int64)[:, None]
+    g = np.arange(4, dtype=np.int64)[None, :]
+    a = e + 2 + 8 * g
+    d = a & ~np.int64(3)
+    spans = [(d, d + 8), (e, e + 2)]
+    spans.append((d + 4 * (1 + (a >> 1 & 1)), d + 8 + 4 * (a >> 1 & 1)) if old
+                 else (a + 6, a + 8))
+    return spans
+
+
+@pytest.mark.parametrize("n_rows,n_blk", [(1, 1), (2, 1), (3, 1), (1, 28), (17, 3), (5, 152)])
+@pytest.mark.parametrize("base", [BASE, BASE + 4])
+def test_q8_gemm_windows_in_bounds(n_rows, n_blk, base):
+    """Every load lies inside the table (its base 4-byte aligned), the blocks
+    past a wave's last one clamped to it; the codes are covered."""
+    end = base + 34 * n_blk * n_rows
+    for r in range(n_rows):
+        spans = q8_gemm_windows(base + 34 * n_blk * r, n_blk)
+        for lo, hi in spans:
+            assert (lo >= base).all() and (hi <= end).all()
+        a = base + 34 * (n_blk * r + np.arange(n_blk)[:, None]) + 2 + 8 * np.arange(4)[None, :]
+        (d0, d1), _, (t0, t1) = spans
+        assert (d0 <= a).all() and (t0 <= d1).all() and (t1 == a + 8).all()
+    last = base + 34 * n_blk * (n_rows - 1)
+    if n_blk * n_rows % 2 and base % 4 == 0:    # the old piece ended 2 bytes past the table
+        assert max(hi.max() for _, hi in q8_gemm_windows(last, n_blk, old=True)) == end + 2
