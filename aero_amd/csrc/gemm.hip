@@ -640,28 +640,34 @@ const Q8Tile kQ8Tiles[] = {
     {4, 4, 3.30, gemm_q8_kernel<4, 4, kQ8Waves>},
 };
 
-// The tile whose rounds of one workgroup a CU cost least. Measured on MI355X,
-// fp32-step GEMM (GEMV below 32 tokens) / this in us: 4864 x 896 at 8 tokens
-// 13.8 / 6.2, 32 30.6 / 8.1, 77 31.8 / 12.1, 512 75.8 / 41.3; 896 x 4864 at
-// 77 116 / 24.7; 4096 x 4096 at 512 171 / 151; 14336 x 4096 at 64 100.5 /
-// 76.6, 512 577 / 522. Error against float64 at 896 columns 5.3e-7 -> 7.6e-8.
-// (AERO_HIP_TUNE gemm_q8_tile=N takes entry N - 1 instead.)
-bool launch_q8(const GemmParams& p, hipStream_t s) {
+// The tile whose rounds of one workgroup a CU cost least (the waves' longest
+// share of a row's blocks apart). Measured on MI355X, fp32-step GEMM (GEMV
+// below 32 tokens) / this in us: 4864 x 896 at 8 tokens 13.8 / 6.4, 32 30.6 /
+// 8.2, 77 31.8 / 12.5, 512 75.8 / 44.5; 896 x 4864 at 77 116 / 25.1; 4096 x
+// 4096 at 512 171 / 152; 14336 x 4096 at 64 100.5 / 77.7, 512 577 / 522. Error
+// against float64 at 896 columns 5.3e-7 -> 7.6e-8.
+const Q8Tile& q8_tile(int64_t n_rows, int64_t n_tok, double* cost = nullptr) {
     const int64_t cus = cu_count();
-    auto wgs = [&](const Q8Tile& t) {
-        return (p.n_rows + 16 * t.nt - 1) / (16 * t.nt) *
-               (((int64_t)p.n_tok + 16 * t.mt - 1) / (16 * t.mt));
-    };
     const Q8Tile* best = nullptr;
     double least = 0.0;
     for (const Q8Tile& t : kQ8Tiles) {
-        if (((int64_t)p.n_tok + 16 * t.mt - 1) / (16 * t.mt) > 65535) continue;
-        const double c = (double)((wgs(t) + cus - 1) / cus) * t.cost;
+        const int64_t tt = (n_tok + 16 * t.mt - 1) / (16 * t.mt);
+        const int64_t wgs = (n_rows + 16 * t.nt - 1) / (16 * t.nt) * tt;
+        // (the last tile takes any call that gemm_dev admits)
+        if (tt > 65535 && &t != std::end(kQ8Tiles) - 1) continue;
+        const double c = (double)((wgs + cus - 1) / cus) * t.cost;
         if (best == nullptr || c < least) {
             best = &t;
             least = c;
         }
     }
+    if (cost != nullptr) *cost = least;
+    return *best;
+}
+
+// (AERO_HIP_TUNE gemm_q8_tile=N takes entry N - 1 instead.)
+bool launch_q8(const GemmParams& p, hipStream_t s) {
+    const Q8Tile* best = &q8_tile(p.n_rows, p.n_tok);
     const int fixed = tune("gemm_q8_tile", 0);
     if (fixed >= 1 && fixed <= (int)(sizeof(kQ8Tiles) / sizeof(kQ8Tiles[0])))
         best = &kQ8Tiles[fixed - 1];
@@ -672,6 +678,12 @@ bool launch_q8(const GemmParams& p, hipStream_t s) {
 }
 
 }  // namespace
+
+double q8_gemm_cost(int64_t n_rows, int64_t n_tok) {
+    double c = 0.0;
+    q8_tile(n_rows, n_tok, &c);
+    return c;
+}
 
 // Called by gemv_dev after its argument checks (W's size and 4-byte
 // alignment, x 16-byte aligned, n_cols a multiple of the block), for

@@ -57,6 +57,10 @@
 
 namespace aero {
 
+bool gemm_dev(int dtype, const uint8_t* w, const float* x, float* y, int64_t n_rows,
+              int64_t n_cols, int64_t rb, int64_t n_tok, hipStream_t s);
+double q8_gemm_cost(int64_t n_rows, int64_t n_tok);
+
 // block sizes of the ggml types (quant.hip)
 int64_t dtype_block_bytes(int t);
 int64_t dtype_block_values(int t);
@@ -1930,13 +1934,23 @@ bool split_gemm_dev(int dtype, const uint8_t* w, const float* x, float* y, int64
         return true;
     if (!split_room_ok(n_rows, n_cols, n_tok, ws_bytes - need)) return true;
     // Q8_0 rows whose super-blocks do not divide (4864 columns: 19) would run
-    // unsplit on a part of the chip: gemm_q8_kernel, whose waves share the
-    // columns, takes them. Measured on MI355X, 896 x 4864, this / that in us:
-    // 16 tokens 45.0 / 16.9, 77 47.6 / 25.5, 256 50.4 / 35.1, 512 52.6 / 51.6.
+    // unsplit on a part of the chip, in about 9 us and 2.1 a super-block
+    // whatever the rows: gemm_q8_kernel, whose waves share the columns, takes
+    // them where its tiles cost less (q8_gemm_cost, us for as many columns).
+    // Measured on MI355X, this / that in us: cost 0.65 (896 x 4864, 16 tokens)
+    // 45.0 / 16.9, 1.15 (4864 x 2816, 12) 28.9 / 16.3, 1.5 (4864 x 4864, 32)
+    // 46.2 / 32.7; 1.95 (11008 x 4864, 16) 45.3 / 47.3, 2.3 (4864 x 4864, 40)
+    // 47.4 / 50.5, 2.5 (11008 x 5888, 32) 53.9 / 61.9. x's pre-pass makes the
+    // line 2.35 from 512 tokens: 896 x 4864 53.3 / 49.8, x 7424 75.9 / 73.6.
+    // (AERO_HIP_TUNE gemm_q8_split=0: this.)
     const int64_t base_wgs = (n_rows + 127) / 128 * (pad_tokens(n_tok) / kTokTile);
-    if (dtype == AERO_DTYPE_Q8_0 && base_wgs < 128 && tune("gemm16_nt", 2) == 2 &&
-        pick_ksplit(base_wgs, (int)(n_cols / 256), n_tok * n_rows * 4, ws_bytes - need) == 1)
-        return true;
+    if (dtype == AERO_DTYPE_Q8_0 && base_wgs < 128 && tune("gemm_q8_split", 1) &&
+        tune("gemm16_nt", 2) == 2 &&
+        pick_ksplit(base_wgs, (int)(n_cols / 256), n_tok * n_rows * 4, ws_bytes - need) == 1 &&
+        q8_gemm_cost(n_rows, n_tok) <= (n_tok >= 512 ? 2.4 : 1.6)) {
+        *ran = true;
+        return gemm_dev(dtype, w, x, y, n_rows, n_cols, rb, n_tok, s);
+    }
     SplitJob j{dtype, x, nullptr, nullptr, nullptr, -1, 0.f, 1, &w, nullptr, 0, &n_rows, &y,
                n_cols, rb, n_tok, ws, {}, ws_bytes};
     if (!split_run(j, s)) return false;

@@ -12,7 +12,7 @@ import pytest
 from conftest import RTOL, golden, rel_to_scale
 from aero_amd import native, ops
 from aero_amd import workloads as W
-from aero_amd.device import DeviceArray as DA, tune_set
+from aero_amd.device import DeviceArray as DA, Event, Plan, tune_set
 
 pytestmark = pytest.mark.gpu
 
@@ -297,3 +297,44 @@ def test_q8_routes_agree(hip, oracle, n_rows, n_cols, n_tok):
         ops.matvec(W.Q8_0, dw, dx, y, n_rows, n_cols, n_tok, split=split)
         assert rel_to_scale(y.numpy(), want) <= RTOL
 
+
+@pytest.mark.parametrize("n_rows,n_cols,n_tok", [
+    (11008, 2816, 12), (4864, 3328, 10), (11008, 4864, 4), (4864, 7424, 77),
+    (896, 4864, 16), (4864, 2816, 12),
+])
+def test_q8_route_is_no_slow_one(hip, n_rows, n_cols, n_tok):
+    """A Q8_0 call with a workspace takes no route that is much slower than
+    another one it could take (GEMV, gemm_q8_kernel, the split GEMM; measured
+    within 1.15, calls sent to a wrong one took 1.4 to 2.1 times)."""
+    rng = np.random.default_rng(1)
+    dw = DA.from_numpy(W.make_table(W.Q8_0, n_rows * n_cols // 32, rng))
+    dx = DA.from_numpy(rng.standard_normal((n_tok, n_cols)).astype(np.float32))
+    y = DA.empty((n_tok, n_rows))
+    print(f"Q8_0 routes {n_rows} x {n_cols}, {n_tok} tokens", flush=True)
+
+    def us(split, **tunes):
+        for key, value in tunes.items():
+            tune_set(key, value)
+        try:
+            plan = Plan()
+            with plan:
+                for _ in range(10):
+                    ops.matvec(W.Q8_0, dw, dx, y, n_rows, n_cols, n_tok, split=split)
+        finally:
+            for key in tunes:
+                tune_set(key, None)
+        best = []
+        for _ in range(6):
+            a, b = Event(), Event()
+            a.record()
+            plan.launch()
+            b.record()
+            b.synchronize()
+            best.append(a.elapsed_ms(b) * 100)
+        plan.destroy()
+        return min(best)
+
+    gemv, gemm = us(False, gemm_min_tokens=1000), us(False, gemm_min_tokens=1)
+    split = us(True, gemm_q8_split=0, gemm_min_tokens=1000)
+    own_ws = us(True)
+    assert own_ws <= 1.3 * min(gemv, gemm, split), (own_ws, gemv, gemm, split)
