@@ -26,6 +26,7 @@ int64_t dtype_block_bytes(int t);
 bool gemm_dev(int dtype, const uint8_t* w, const float* x, float* y, int64_t n_rows,
               int64_t n_cols, int64_t rb, int64_t n_tok, hipStream_t s);
 int64_t split_gemm_workspace(int dtype, int64_t n_cols, int64_t n_tok);
+double q8_gemm_cost(int64_t n_rows, int64_t n_tok);
 bool split_tokens_ok(int64_t n_tok, int64_t n_rows, int64_t n_cols);
 bool split_gemm_dev(int dtype, const uint8_t* w, const float* x, float* y, int64_t n_rows,
                     int64_t n_cols, int64_t rb, int64_t n_tok, void* ws, int64_t ws_bytes,
@@ -1617,6 +1618,33 @@ bool lanes64_ok(int dtype, const uint8_t* w, int64_t rb, int64_t n_rows, int64_t
     return w_bytes >= end + ((16 - (end & 15)) & 15);
 }
 
+namespace {
+
+// Whether gemm_q8_kernel serves a Q8_0 call of 5 to 31 tokens in less time
+// than the GEMV. Measured on MI355X, GEMV / GEMM in us. Up to one GEMV step
+// (4096 columns, 4 tokens a launch): 896 columns, 4864 rows at 4 tokens 7.2 /
+// 6.3, 5 10.8 / 6.3; 1792, 128 rows at 5 8.7 / 6.5; 2048, 11008 rows at 6 22.6
+// / 25.0, 7 28.6 / 25.1, 128 rows at 6 9.4 / 9.2; 4096, 1024 rows at 8 11.9 /
+// 17.2, 12 17.5 / 18.3. Longer rows take 2 tokens a GEMV launch, of about 3.2
+// us and 1.6 a step and 1400 rows; the GEMM's waves take 1.1 times
+// q8_gemm_cost an eighth of the blocks, 1.4 where the columns are a multiple
+// of 2048 (the rows' blocks then meet in the same cache channels): 896 rows at
+// 5 tokens of 4864 columns 18.0 / 14.3, 7424 18.2 / 20.5, 8192 18.3 / 29.2,
+// 28672 41.2 / 96.3; 4864 rows of 7424 45.9 / 34.6, of 8192 49.3 / 50.4.
+bool q8_gemm_ok(int64_t n_tok, int64_t n_rows, int64_t n_cols) {
+    if (n_tok < 5) return false;
+    if (n_cols <= kStepCols) return n_tok >= (n_cols <= 1792 ? 5 : n_cols <= 2048 ? 7 : 13);
+    const double steps = (double)((n_cols + kStepCols - 1) / kStepCols);
+    const double gemv = (0.5 * (double)n_tok + (n_tok & 1 ? 0.2 : 0.0)) *
+                        (3.2 + 1.6 * steps * std::max(1.0, (double)n_rows / 1400.0));
+    const double gemm = 1.5 + (n_cols % 2048 == 0 ? 1.4 : 1.1) *
+                                  (double)((n_cols / 32 + 7) / 8) * q8_gemm_cost(n_rows, n_tok);
+    return gemm < gemv;
+}
+
+}  // namespace
+
+
 bool gemv_dev(int dtype, const uint8_t* w, int64_t w_bytes, const float* x, float* y,
               int64_t n_rows, int64_t n_cols, int64_t n_tok, hipStream_t s, void* ws,
               int64_t ws_bytes) {
@@ -1650,22 +1678,15 @@ bool gemv_dev(int dtype, const uint8_t* w, int64_t w_bytes, const float* x, floa
     // several tokens: the matrix-core GEMMs. The split-x fp16 one when a
     // workspace is given and the type has it (from 5-16 tokens by the
     // matrix size, split_tokens_ok), else the fp32 one from 32 tokens (W
-    // once per 64), or Q8_0's bf16 one from 5 where the GEMV takes rows of up
-    // to half a step or more than one, from 13 where it takes 4 tokens a
-    // launch of one-step rows. Measured on MI355X, GEMV / GEMM in us: 4864 x
-    // 896 at 4 tokens 7.2 / 6.3, 8 13.8 / 6.2; 896 x 4864 at 4 12.8 / 13.9, 5
-    // 17.3 / 13.9; 512 x 2048 at 5 9.0 / 9.0, 8 11.7 / 9.7; 1024 x 4096 at 8
-    // 11.9 / 17.2, 12 17.5 / 18.3; 14336 x 4096 at 5 39.9 / 52.5.
+    // once per 64), or Q8_0's bf16 one from fewer (q8_gemm_ok).
     if (ws != nullptr && n_tok <= (int64_t)1 << 30 && split_tokens_ok(n_tok, n_rows, n_cols)) {
         bool ran = false;
         if (!split_gemm_dev(dtype, w, x, y, n_rows, n_cols, rb, n_tok, ws, ws_bytes, s, &ran))
             return false;
         if (ran) return true;
     }
-    const int min_tok = dtype != AERO_DTYPE_Q8_0 ? 32
-                        : 2 * n_cols <= kStepCols || n_cols > kStepCols ? 5 : 13;
-    if (n_tok >= tune("gemm_min_tokens", min_tok) &&
-        n_tok <= (int64_t)1 << 30)
+    const bool q8 = dtype == AERO_DTYPE_Q8_0 && q8_gemm_ok(n_tok, n_rows, n_cols);
+    if (n_tok >= tune("gemm_min_tokens", q8 ? 5 : 32) && n_tok <= (int64_t)1 << 30)
         return gemm_dev(dtype, w, x, y, n_rows, n_cols, rb, n_tok, s);
     if (lanes64_ok(dtype, w, rb, n_rows, w_bytes) && tune("gemv_lanes64", 1)) {
         const bool pipe = n_cols > kStepCols;

@@ -299,13 +299,15 @@ def test_q8_routes_agree(hip, oracle, n_rows, n_cols, n_tok):
 
 
 @pytest.mark.parametrize("n_rows,n_cols,n_tok", [
-    (11008, 2816, 12), (4864, 3328, 10), (11008, 4864, 4), (4864, 7424, 77),
+    (11008, 2816, 12), (4864, 3328, 10), (11008, 4864, 4), (4864, 7424, 77),   # workspace
     (896, 4864, 16), (4864, 2816, 12),
+    (11008, 2048, 5), (896, 8192, 5), (128, 28672, 8), (896, 4864, 5), (4864, 896, 5),
 ])
 def test_q8_route_is_no_slow_one(hip, n_rows, n_cols, n_tok):
     """A Q8_0 call with a workspace takes no route that is much slower than
-    another one it could take (GEMV, gemm_q8_kernel, the split GEMM; measured
-    within 1.15, calls sent to a wrong one took 1.4 to 2.1 times)."""
+    another one it could take (GEMV, gemm_q8_kernel, the split GEMM), one
+    without none that is much slower than the GEMV (measured within 1.15; calls
+    sent to a wrong one took 1.4 to 2.5 times)."""
     rng = np.random.default_rng(1)
     dw = DA.from_numpy(W.make_table(W.Q8_0, n_rows * n_cols // 32, rng))
     dx = DA.from_numpy(rng.standard_normal((n_tok, n_cols)).astype(np.float32))
@@ -336,5 +338,6 @@ def test_q8_route_is_no_slow_one(hip, n_rows, n_cols, n_tok):
 
     gemv, gemm = us(False, gemm_min_tokens=1000), us(False, gemm_min_tokens=1)
     split = us(True, gemm_q8_split=0, gemm_min_tokens=1000)
-    own_ws = us(True)
+    own, own_ws = us(False), us(True)
+    assert own <= 1.3 * gemv, (own, gemv, gemm)
     assert own_ws <= 1.3 * min(gemv, gemm, split), (own_ws, gemv, gemm, split)
