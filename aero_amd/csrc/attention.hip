@@ -1296,27 +1296,34 @@ bool attn_plan(int64_t n_q, int64_t n_head, int64_t n_head_kv, int64_t head_dim,
 
 // Whether a call that attn_mfma_kernel would take as one chunk goes to
 // attn_split_kernel: fp32 caches, and enough workgroups (128 query vectors of
-// a kv head each, one a CU) that the chip is half full, or more than a
-// quarter full over long key ranges, where the split of the keys is paid back.
-// Measured on MI355X, fp32-step kernel / this one in us, causal prompts
-// unless noted: 8 kv heads of dim 128, 32 heads: 104 workgroups (400 tokens)
-// 35.0 / 36.8, after 1000 cached keys 141 / 90; 176 (700 tokens) 76.0 / 52.7;
-// 512 (2048 tokens) 463 / 150; dim 64: 104 workgroups 19.4 / 25.1, after 1000
-// keys 84.6 / 51.7; 176: 44.8 / 33.4. Two kv heads of dim 64, 14 heads, 78
-// workgroups: 25.7 / 31.2, after 1000 keys 69.8 / 60.1. Dim 256, 88
-// workgroups: 152 / 179 (1400 tokens, 700 keys a query), after 1000 keys
-// 309 / 294 and in a window of 1024 208 / 150. Below 72 workgroups the
-// fp32-step kernel, which also splits the keys, is the faster one for most
-// sizes (64 workgroups of dim 128, 256 tokens: 18.2 / 26.8).
+// a kv head each, one a CU) that the chip is half full (150 at head dim 64
+// where a query keeps fewer than 200 keys, which pay for less of the
+// prologue), or more than a quarter full over long key ranges, where the split
+// of the keys is paid back; not the latter with key positions, where every key
+// is walked and each tile masked. Measured on MI355X, fp32-step kernel / this one in us, causal
+// prompts unless noted: 8 kv heads of dim 128, 32 heads: 104 workgroups (400
+// tokens) 35.0 / 36.8, after 1000 cached keys 141 / 90; 176 (700 tokens) 76.0 /
+// 53.5; 512 (2048 tokens) 463 / 150; dim 64: 104 workgroups 19.4 / 25.1, after
+// 1000 keys 84.6 / 51.7; 176: 44.8 / 33.4; 128 in a window of 128 21.2 / 24.0.
+// Two kv heads of dim 64, 14 heads, 78 workgroups: 25.7 / 31.2, after 1000
+// keys 69.8 / 60.1. Dim 256, 88 workgroups: 152 / 179 (1400 tokens, 700 keys a
+// query), after 1000 keys 309 / 294 and in a window of 1024 208 / 150; shuffled
+// keys after 4000 909 / 1012.
+// Fewer workgroups stay with the fp32-step kernel, which also splits the keys.
+// A line on their number is not the best for all: that kernel's time rises in
+// steps with its own grid (64 of dim 128, 256 tokens: 18.2 / 26.8, but 32, 128
+// tokens: 26.5 / 19.3; 44 of dim 64, 14 / 2 heads, 400 tokens: 37.0 / 23.8; 50
+// of dim 256, 16 / 2 heads, 400 tokens: 96.8 / 65.5).
 void plan_split(int64_t n_q, int64_t n_head, int64_t n_head_kv, int64_t head_dim, int64_t n_kv,
-                int window, int kv_dt, AttnPlan& pl) {
+                int window, int kv_dt, bool kpos, AttnPlan& pl) {
     const int use = tune("attn_split", 1);   // 2: whatever the sizes
     const int64_t grid_z = (n_q * (n_head / n_head_kv) + kSplitVecs - 1) / kSplitVecs;
     const int64_t wgs = n_head_kv * grid_z;
     int64_t mean = std::max<int64_t>(n_kv - n_q / 2, 1);   // keys a query, causal
     if (window > 0) mean = std::min<int64_t>(mean, window);
     if (!pl.mfma || kv_dt != 0 || use == 0 ||
-        (use == 1 && (pl.n_chunks != 1 || !(wgs >= 128 || (wgs >= 72 && mean >= 1000)))) ||
+        (use == 1 && (pl.n_chunks != 1 || !(wgs >= (head_dim == 64 && mean < 200 ? 150 : 128) ||
+                                            (wgs >= 72 && mean >= 1000 && !kpos)))) ||
         // (32-bit key indices and offsets within a key tile)
         n_kv >= (int64_t(1) << 30) || n_head_kv * head_dim * 4 * 128 >= (int64_t(1) << 31))
         return;
@@ -1459,7 +1466,7 @@ bool attention_dev(const float* q, int kv_dt, const void* k, const float* k_scal
         set_error("attention: grid too large");
         return false;
     }
-    plan_split(n_q, n_head, n_head_kv, head_dim, n_kv, window, kv_dt, pl);
+    plan_split(n_q, n_head, n_head_kv, head_dim, n_kv, window, kv_dt, kpos != nullptr, pl);
     AttnParams p{q, k, k_scale, v, v_scale, out, static_cast<float*>(workspace), qpos, kpos,
                  n_q, n_head, n_head_kv, head_dim, value_dim, n_kv,
                  (int)(n_head / n_head_kv), window, scale, pl.chunk_len, pl.n_chunks};

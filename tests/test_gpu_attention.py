@@ -599,24 +599,41 @@ def test_split_redo(split_always, T, H, HK, D, S, window, kpos):
     assert ms[1] <= 10 * ms[0], ms
 
 
-def test_split_rule_matches_general(hip):
-    """Calls on both sides of the rule's line agree with the fp32-step kernel,
-    a window, shuffled keys and cached prefixes among them."""
+@pytest.mark.parametrize("T,H,HK,D,S,window,kpos,split", [
+    (255, 64, 8, 128, 255, 0, False, True),      # 128 workgroups, 128 keys a query
+    (239, 64, 8, 128, 239, 0, False, False),     # 120
+    (508, 32, 8, 64, 508, 0, False, True),       # 128 over 255
+    (600, 32, 8, 64, 700, 128, False, True),     # 152 in a window of 128
+    (508, 32, 8, 64, 700, 128, False, False),    # 128 in a window of 128
+    (480, 32, 8, 64, 480, 0, False, False),      # 120 over 241
+    (255, 32, 8, 64, 1300, 0, False, False),     # 64 over 1173
+    (288, 32, 8, 64, 1300, 0, False, True),      # 72
+    (284, 32, 8, 128, 1100, 0, False, False),    # 72 over 959
+    (600, 14, 2, 64, 1700, 0, True, False),      # 66, shuffled keys
+    (700, 16, 2, 256, 1700, 0, True, False),     # 88 over 1350, shuffled keys
+    (700, 16, 2, 256, 1700, 0, False, True),
+    (1024, 16, 2, 256, 1024, 300, True, True),   # 128, shuffled keys in a window
+])
+def test_split_rule_matches_general(hip, T, H, HK, D, S, window, kpos, split):
+    """Calls on both sides of the rule's lines run the kernel that they are
+    meant to (both are deterministic: their bits tell) and agree with the
+    other, a window, shuffled keys and cached prefixes among them."""
     rng = np.random.default_rng(3)
-    for T, H, HK, D, S, window, kpos in [(256, 64, 8, 128, 256, 0, False),
-                                         (255, 32, 8, 64, 1300, 0, False),
-                                         (600, 14, 2, 64, 1700, 0, True),
-                                         (1024, 16, 2, 256, 1024, 300, False)]:
-        q, k, v = rand_qkv(rng, T, H, HK, D, D, S)
-        qpos = np.arange(S - T, S, dtype=np.int32)
-        kp = rng.permutation(S).astype(np.int32) if kpos else None
-        got = gpu_attention(q, k, v, 1.0 / np.sqrt(D), qpos=qpos, kpos=kp, window=window)
-        tune_set("attn_split", 0)
+    q, k, v = rand_qkv(rng, T, H, HK, D, D, S)
+    qpos = np.arange(S - T, S, dtype=np.int32)
+    kp = rng.permutation(S).astype(np.int32) if kpos else None
+    print(f"attention rule T={T} H={H} HK={HK} D={D} S={S} window={window}", flush=True)
+    out = []
+    for use in (None, 0, 2):
+        tune_set("attn_split", use)
         try:
-            want = gpu_attention(q, k, v, 1.0 / np.sqrt(D), qpos=qpos, kpos=kp, window=window)
+            out.append(gpu_attention(q, k, v, 1.0 / np.sqrt(D), qpos=qpos, kpos=kp,
+                                     window=window))
         finally:
             tune_set("attn_split", None)
-        assert rel_to_scale(got, want) <= RTOL
+    assert not bits_equal(out[1], out[2])
+    assert bits_equal(out[0], out[2 if split else 1])
+    assert rel_to_scale(out[2], out[1]) <= RTOL
 
 
 def test_split_output_past_2_32_elements(hip, oracle):
