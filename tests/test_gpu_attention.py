@@ -444,8 +444,10 @@ def test_split_vs_oracle(split_always, oracle, T, H, HK, D, S, window, kpos):
 @pytest.mark.parametrize("where", ["q", "k", "v"])
 def test_split_non_finite(split_always, oracle, D, bad, where):
     """A non-finite or huge operand touches the queries that keep it and no
-    other: those agree with the oracle's result without it; where the
-    fp32-step kernel gives the touched ones a finite row, so does this one."""
+    other: those agree with the oracle's result without it. The touched ones
+    are the fp32-step kernel's where its row is finite; where it is not, the
+    split's is not either, and each element is the NaN or infinity that the
+    fp32-step kernel gives it."""
     rng = np.random.default_rng(D)
     T, H, HK, S = 70, 4, 2, 100
     q, k, v = rand_qkv(rng, T, H, HK, D, D, S)
@@ -468,6 +470,10 @@ def test_split_non_finite(split_always, oracle, D, bad, where):
         if np.isfinite(general[t, h]).all():
             assert rel_to_scale(got[t, h].astype(np.float64),
                                 general[t, h].astype(np.float64)) <= RTOL
+        else:
+            assert np.array_equal(np.isnan(got[t, h]), np.isnan(general[t, h])), (t, h)
+            inf = np.isinf(general[t, h])
+            assert np.array_equal(got[t, h][inf], general[t, h][inf]), (t, h)
 
 
 @pytest.mark.parametrize("D", [64, 128, 256])
