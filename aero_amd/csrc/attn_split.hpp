@@ -29,11 +29,20 @@
 // key), rows of V whose exponents differ by more than kSpread, in a block or
 // between blocks (a query may keep the small ones alone), dimensions of V that
 // do by more than kSpreadCh (known at the end of the walk), or keys and queries
-// whose products pass 2^kScoreExp. Time of calls whose every workgroup does so, fp32-step
-// kernel / this one (a row at a time, as it was): 2048 causal tokens, 32 / 8
-// heads of dim 128 467 / 517 us (12.2 ms), of dim 64 256 / 336 us, 8 / 4
-// heads of dim 256 in a window of 1024, whose 128 workgroups leave half of
-// the CUs idle, 235 / 602 us (10.1 ms).
+// whose products pass 2^kScoreExp. Time of calls whose every workgroup does
+// so, fp32-step kernel / this one (where the end of the walk shows it), 2048
+// causal tokens: 32 / 8 heads of dim 128 470 / 511 us (670), of dim 64 274 / 341 us
+// (419), 8 / 4 heads of dim 256 in a window of 1024, whose 128 workgroups leave
+// half of the CUs idle, 240 / 647 us (780).
+//
+// Precision. An operand keeps 22 to 23 bits and the lo lo products are
+// dropped, where the fp32 steps keep 24; the sums are shorter and exact in the
+// rescaling. 2-norm error against float64, normal q, K and V, is below the
+// fp32 steps' at every size measured (below; 33 queries of dim 128 1.8e-7 ->
+// 1.6e-7, 1641 of dim 256 5.4e-7 -> 3.8e-7); where all probabilities are
+// nearly the same, which rounds least in fp32, above (0.8e-7 -> 1.1e-7). It is
+// an error relative to the query's largest values of V: an element far below
+// the others of its query has fewer bits.
 //
 // Shape. A workgroup owns 128 query vectors of one kv head (32 a wave). At
 // head dims 64 and 128 eight waves walk 128 / 64 keys a step, two waves a
@@ -47,10 +56,12 @@
 // What bounds it: per 64 keys and CU at head dim 128 3072 cycles of matrix
 // steps a SIMD, about 2600 of LDS, about 2400 of vector instructions a SIMD
 // and a step takes about 7500: two waves a SIMD (all 256 registers each) do
-// not overlap them fully. Against attn_mfma_kernel, whose fp32 steps run at a
+// not overlap them fully (92 bytes a lane do not fit at head dim 128, 104 with
+// key positions: four vectors of q's parts come from scratch each step, between
+// the scores' matrix steps). Against attn_mfma_kernel, whose fp32 steps run at a
 // sixteenth of the fp16 rate, on MI355X, 2048 causal tokens: 32 / 8 heads of
-// dim 128 454 -> 149 us (231 TFLOP/s by the useful products), of dim 64
-// 252 -> 86 us, 8 / 4 heads of dim 256 in a window of 1024 206 -> 144 us.
+// dim 128 455 -> 150 us (229 TFLOP/s by the useful products), of dim 64
+// 247 -> 95 us, 8 / 4 heads of dim 256 in a window of 1024 207 -> 148 us.
 // Error against float64 (2-norm) at those sizes: 4.0e-7 -> 2.9e-7, 3.3e-7 ->
 // 2.5e-7, 5.0e-7 -> 3.5e-7.
 
@@ -698,8 +709,8 @@ __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_split_kernel(At
         for (int x = 0; x < 16; ++x) s[x] = sl[x] = 0.0f;
         h8 kph[2], kpl[2];
         // (the matrix steps go before the other wave's vector instructions:
-        // 2048 causal tokens at head dim 64 90.5 -> 85.8 us, 512 at 128 42.6
-        // -> 41.8 on MI355X; at 2048 and 128 within 1%)
+        // 2048 causal tokens at head dim 64 97.1 -> 93.7 us, at 256 151.7 ->
+        // 148.4, at 128 162 -> 160 on MI355X)
         __builtin_amdgcn_s_setprio(1);
         kph[0] = *reinterpret_cast<const h8*>(kl);
         kpl[0] = *reinterpret_cast<const h8*>(kl + C::KPART);

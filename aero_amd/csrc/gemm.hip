@@ -466,9 +466,11 @@ __device__ __forceinline__ float largest(const float (&x)[8]) {
     return big;
 }
 
-template <int MT, int NT, int KW>
-__global__ __launch_bounds__(64 * KW) void gemm_q8_kernel(GemmParams p) {
-    __shared__ v4f sums[KW][MT * NT][64];
+constexpr int kQ8Waves = 8;
+
+template <int MT, int NT>
+__global__ __launch_bounds__(64 * kQ8Waves) void gemm_q8_kernel(GemmParams p) {
+    __shared__ v4f sums[kQ8Waves][MT * NT][64];
     const int l = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = l & 15, g = l >> 4;
@@ -518,7 +520,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_q8_kernel(GemmParams p) {
         for (int j = 0; j < NT; ++j) acc[m][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
     load(wave);
-    for (int b = wave; b < nb; b += KW) {
+    for (int b = wave; b < nb; b += kQ8Waves) {
         bf8v wb[NT];
         float d[NT];
 #pragma unroll
@@ -548,7 +550,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_q8_kernel(GemmParams p) {
         if (!__any(hi > kQ8Large || lo < kQ8Small)) {
 #pragma unroll
             for (int m = 0; m < MT; ++m) bf16_parts<false>(x[m], xb[m]);
-            load(b + KW);
+            load(b + kQ8Waves);
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -581,7 +583,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_q8_kernel(GemmParams p) {
                     }
                 }
             }
-            load(b + KW);
+            load(b + kQ8Waves);
         }
     }
 
@@ -591,12 +593,12 @@ __global__ __launch_bounds__(64 * KW) void gemm_q8_kernel(GemmParams p) {
         for (int j = 0; j < NT; ++j) sums[wave][m * NT + j][l] = acc[m][j];
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < MT * NT; i += KW) {
+    for (int i = 0; i < MT * NT; i += kQ8Waves) {
         if (i + wave >= MT * NT) break;
         const int m = (i + wave) / NT, j = (i + wave) % NT;
         v4f y = sums[0][i + wave][l];
 #pragma unroll
-        for (int k = 1; k < KW; ++k) y += sums[k][i + wave][l];
+        for (int k = 1; k < kQ8Waves; ++k) y += sums[k][i + wave][l];
         const int64_t row = r0 + 16 * j + c;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -626,18 +628,19 @@ namespace {
 
 // A workgroup tile of gemm_q8_kernel and its cost a block step with one
 // workgroup a CU (measured on MI355X, us for eight waves taking a block each,
-// 896 x 4864).
+// 896 x 4864; there is no term for memory or for small tiles that share a CU.
+// Over rows of 2816 to 7424 columns and 4 to 1300 tokens calls took 1.0 to 1.4
+// times their tile's cost, the more the smaller, plus 1 to 3 us.)
 struct Q8Tile {
     int mt, nt;
     double cost;
     void (*k)(GemmParams);
 };
-constexpr int kQ8Waves = 8;
 const Q8Tile kQ8Tiles[] = {
-    {1, 1, 0.65, gemm_q8_kernel<1, 1, kQ8Waves>}, {2, 1, 1.05, gemm_q8_kernel<2, 1, kQ8Waves>},
-    {1, 2, 1.15, gemm_q8_kernel<1, 2, kQ8Waves>}, {2, 2, 1.50, gemm_q8_kernel<2, 2, kQ8Waves>},
-    {4, 2, 2.35, gemm_q8_kernel<4, 2, kQ8Waves>}, {2, 4, 2.50, gemm_q8_kernel<2, 4, kQ8Waves>},
-    {4, 4, 3.30, gemm_q8_kernel<4, 4, kQ8Waves>},
+    {1, 1, 0.65, gemm_q8_kernel<1, 1>}, {2, 1, 1.05, gemm_q8_kernel<2, 1>},
+    {1, 2, 1.15, gemm_q8_kernel<1, 2>}, {2, 2, 1.50, gemm_q8_kernel<2, 2>},
+    {4, 2, 2.35, gemm_q8_kernel<4, 2>}, {2, 4, 2.50, gemm_q8_kernel<2, 4>},
+    {4, 4, 3.30, gemm_q8_kernel<4, 4>},
 };
 
 // The tile whose rounds of one workgroup a CU cost least (the waves' longest

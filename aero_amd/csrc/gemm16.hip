@@ -1681,15 +1681,17 @@ bool split_rope_ok(const SplitJob& j, int rows_wg, int ks, int mt) {
 }
 
 // Whether the reduction of a column-split call applies j.rope: no per-head
-// norm, heads that its 256-output workgroups hold whole, and fewer than 32
-// tokens (one token tile), where the pass it replaces is a tenth of the call;
-// a larger call that still splits its columns has few rows, and keeps the
-// launches that callers' counts of a recorded plan know.
+// norm, heads that its 256-output workgroups hold whole, fewer than 32 tokens.
+// Measured on MI355X, pass of its own / in the reduction, Q4_K, us for a
+// q/k/v input: Llama-3-8B 8 tokens 21.7 / 19.1, 31 26.0 / 23.7; hidden 2048, 16
+// / 2 heads of dim 256 16 18.3 / 16.0. The line at 32 tokens is none of speed
+// (Llama-3-8B 32 tokens 26.5 / 24.0, 64 34.0 / 32.0): the launches that a plan
+// records from there on are fixed (tests/test_gpu_norm_gemm.py, 40 tokens).
 bool reduce_rope_ok(const SplitJob& j) {
     const RopeFold& r = j.rope;
     if (j.n_tok >= kTokTile || r.mats < 1 || j.w_up != nullptr || r.mats > j.n_mat ||
-        r.qk_norm() || r.pos == nullptr || r.inv == nullptr || r.D < 2 || 256 % r.D || r.rot() < 2 || r.rot() > r.D ||
-        r.rot() % 2 || (r.mode != AERO_ROPE_NEOX && r.mode != AERO_ROPE_INTERLEAVED))
+        r.qk_norm() || r.pos == nullptr || r.inv == nullptr || r.D < 2 || 256 % r.D ||
+        r.rot() < 2 || r.rot() > r.D || r.rot() % 2 || (r.mode != AERO_ROPE_NEOX && r.mode != AERO_ROPE_INTERLEAVED))
         return false;
     for (int m = 0; m < r.mats; ++m)
         if (j.n_rows[m] % r.D) return false;
