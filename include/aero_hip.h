@@ -340,8 +340,10 @@ int aero_hip_dequant(int dtype, const uint8_t* raw, int64_t raw_len, float* out,
  * y[t*n_rows + r] = sum_c W[r, c] * x[t*n_cols + c] for t < n_tok, W =
  * n_rows rows of (n_cols/bv)*bb bytes of type dtype (Q8_0, Q4_K, Q5_K, Q6_K,
  * IQ4_XS; w_bytes >= that, base 4-byte aligned), x fp32 16-byte aligned.
- * n_cols must be a multiple of the block size. Sums run in a different order
- * from the reference's serial loop (equal to ~1e-6 of the output scale). */
+ * n_cols must be a multiple of the block size. From 32 tokens on fp32 matrix
+ * steps; Q8_0, often from 5, on bf16 ones with x in three parts (all 24 bits).
+ * Sums run in a different order from the reference's serial loop (equal to
+ * ~1e-6 of the output scale). */
 int aero_hip_matvec(int dtype, const uint8_t* w, int64_t w_bytes, const float* x,
                     float* y, int64_t n_rows, int64_t n_cols, int64_t n_tok,
                     void* stream);
@@ -356,7 +358,9 @@ int aero_hip_matvec(int dtype, const uint8_t* w, int64_t w_bytes, const float* x
  * n_tok) bytes (W 16-byte aligned), the GEMM runs on the fp16 matrix cores
  * with x split into two fp16 parts per token and 256 columns (22
  * significant bits of x, exact products, fp32 sums; ws holds the parts);
- * otherwise it is aero_hip_matvec. Below 16 tokens the split GEMM is taken
+ * Q8_0 rows whose 256-column groups do not divide over more workgroups take
+ * aero_hip_matvec's bf16 matrix steps where those are faster; otherwise it is
+ * aero_hip_matvec. Below 16 tokens the split GEMM is taken
  * only when ws also holds aero_hip_split_partials_bytes for its column
  * splits (unsplit it is slower than the GEMV there). Calls sharing one
  * workspace must be ordered on one stream. */
